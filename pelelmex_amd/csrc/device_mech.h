@@ -19,7 +19,7 @@ struct RxRec {
   double lnA0, beta0, Ta0;    // low-pressure limit (falloff)
   double troe[4];             // a, T***, T*, T**
   double effd;                // default collision efficiency
-  double pad;
+  int32_t qoff, pad;          // rate row of the reaction in its chunk (records of the block kernels), unused
   int32_t info;               // type | rev << 4 | nreac << 8 | nprod << 12 | ntroe << 16
   int32_t reac;               // three 8-bit species slots
   int32_t prod;               // three 8-bit species slots

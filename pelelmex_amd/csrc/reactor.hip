@@ -19,6 +19,7 @@
 
 #include "../../include/pele_reactor_capi.h"
 #include "surrogate_kernel.h"
+#include "block_rates.h"
 #include "chem_boxes.h"
 #include "eos_kernel.h"
 #include "mech/drm19.h"
@@ -61,6 +62,7 @@ using EvalLaunch = hipError_t (*)(int mode, const unsigned char* blob, int blob_
                                   hipStream_t st);
 using Occ = hipError_t (*)(int* nb, int block, size_t shmem);
 using RateLaunch = hipError_t (*)(const prk::RateParams&, int blocks, int block, size_t shmem, hipStream_t);
+using BlockRateLaunch = hipError_t (*)(const prk::RateParams&, const prk::BlockTabs&, int cus, hipStream_t);
 using TrustLaunch = hipError_t (*)(const prk::TrustParams&, int blocks, int block, size_t shmem, hipStream_t);
 using FeatLaunch = hipError_t (*)(const prk::FeatParams&, hipStream_t);
 using PrepLaunch = hipError_t (*)(const prk::PrepParams&, int blocks, int block, size_t shmem, hipStream_t);
@@ -88,6 +90,22 @@ hipError_t eval_t(int mode, const unsigned char* blob, int blob_bytes, int neff,
 template <int N, int R, int G>
 hipError_t rate_t(const prk::RateParams& P, int blocks, int block, size_t shmem, hipStream_t st) {
   hipLaunchKernelGGL((prk::rate_kernel<N, R, G>), dim3(blocks), dim3(block), shmem, st, P);
+  return hipGetLastError();
+}
+
+template <int N, int R, int G>
+constexpr size_t rates_block_shmem() {
+  using L = prk::RateLds<N, R, G>;
+  return 8 * (size_t)(L::cg_doubles + L::q_doubles + L::sc_doubles) + N * sizeof(prk::SpRec);
+}
+
+template <int N, int R, int G>
+hipError_t rates_block_t(const prk::RateParams& P, const prk::BlockTabs& tab, int cus, hipStream_t st) {
+  constexpr size_t shmem = rates_block_shmem<N, R, G>();
+  static_assert(shmem <= 163840, "LDS of one CU");
+  const long rounds = (P.ncells + 63) / 64, cap = (long)cus * (long)(163840 / shmem);
+  hipLaunchKernelGGL((prk::rates_block_kernel<N, R, G>), dim3((unsigned)(rounds < cap ? rounds : cap)), dim3(64 * G),
+                     shmem, st, P, tab);
   return hipGetLastError();
 }
 
@@ -172,6 +190,33 @@ const Variant kVariants[] = {
     PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 3),
 };
 
+// Lanes per cell of the block kernels (block_rates.h): a quad up to 32 components, 8 lanes above.
+constexpr int block_lanes(int n) { return n <= 32 ? 4 : 8; }
+
+// The block kernels of each mechanism (64 cells per block, block_lanes lanes per cell).
+struct BlockOps {
+  const char* mech;
+  int waves, nchunk;
+  BlockRateLaunch rates;
+};
+
+#define PR_BLOCK_OPS(NAME, NS, NR) \
+  {NAME, block_lanes(NS + 1), prk::BlockCell<NS, NR, block_lanes(NS + 1)>::NCHUNK, \
+   &rates_block_t<NS, NR, block_lanes(NS + 1)>}
+
+const BlockOps kBlockOps[] = {
+    PR_BLOCK_OPS("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR),
+    PR_BLOCK_OPS("drm19", PR_DRM19_NSP, PR_DRM19_NR),
+    PR_BLOCK_OPS("syn53", PR_SYN53_NSP, PR_SYN53_NR),
+    PR_BLOCK_OPS("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR),
+};
+
+const BlockOps* find_block_ops(const char* mech) {
+  for (const BlockOps& b : kBlockOps)
+    if (std::strcmp(b.mech, mech) == 0) return &b;
+  return nullptr;
+}
+
 const Variant* find_variant(const char* mech, int G, int W = 0) {
   for (const Variant& v : kVariants)
     if (std::strcmp(v.mech, mech) == 0 && (G == 0 || v.G == G) && (W == 0 || v.waves == W)) return &v;
@@ -231,7 +276,7 @@ std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
     o.Ta0 = m->low[3 * r + 2];
     for (int c = 0; c < 4; ++c) o.troe[c] = m->troe[4 * r + c];
     o.effd = m->eff_dflt[r];
-    o.pad = 0.0;
+    o.qoff = o.pad = 0;
     o.info = m->rtype[r] | (m->rev[r] << 4) | (m->nreac[r] << 8) | (m->nprod[r] << 12) | (m->ntroe[r] << 16);
     int ra = 0, pa = 0;
     for (int s = 0; s < m->nreac[r]; ++s) ra |= m->reac[3 * r + s] << (8 * s);
@@ -268,6 +313,81 @@ std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
   kblk[m->nsp] = nb;
   blk[nb] = m->ninc;
   return b;
+}
+
+// Tables of the block kernels' cells layout for a mechanism: reaction records grouped by chunk of
+// consecutive reactions and by wavefront (the heaviest first, each to the wavefront with the least
+// work so far, so the wavefronts reach the chunk's barrier together), and the incidence lists cut
+// into pieces of one gather block and one chunk. Offsets of the four sections go to off[].
+std::vector<unsigned char> pack_block_tabs(const pr_mech_t* m, const std::vector<unsigned char>& blob, int waves,
+                                           int nchunk, size_t off[4]) {
+  const prk::BlobLayout L = prk::blob_layout(m->nsp, m->nr, m->neff, m->ninc);
+  const auto* rx0 = reinterpret_cast<const prk::RxRec*>(blob.data() + L.off_rx);
+  const auto* incq = reinterpret_cast<const int*>(blob.data() + L.off_incq);  // 8 x slot of each entry's reaction
+  std::vector<int> slot_of(m->nr);
+  for (int e = 0; e < m->ninc; ++e) slot_of[m->inc_r[e]] = incq[e] / (int)sizeof(double);
+  const int qrows = (m->nr + nchunk - 1) / nchunk;
+  std::vector<prk::RxRec> rx;
+  std::vector<int32_t> rrange(1, 0), prange(1, 0);
+  std::vector<prk::GatherPiece> pieces;
+  for (int c = 0; c < nchunk; ++c) {
+    const int r0 = c * qrows, r1 = std::min(m->nr, r0 + qrows);
+    auto cost = [&](int r) {  // operations of a rate, roughly: exponentials, logarithms and divisions
+      const int t = m->rtype[r];
+      double w = 35.0 + (m->rev[r] ? 30.0 : 0.0);
+      if (t != PR_RX_ELEM) w += 10.0 + 5.0 * (m->eff_start[r + 1] - m->eff_start[r]);
+      if (t >= PR_RX_LINDEMANN) w += 65.0;
+      if (t == PR_RX_TROE) w += 200.0 + (m->ntroe[r] == 4 ? 28.0 : 0.0);
+      return w;
+    };
+    std::vector<int> order;
+    for (int r = r0; r < r1; ++r) order.push_back(r);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
+    std::vector<std::vector<int>> mine(waves);
+    std::vector<double> load(waves, 0.0);
+    for (int r : order) {
+      const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+      mine[w].push_back(r);
+      load[w] += cost(r);
+    }
+    for (int w = 0; w < waves; ++w) {
+      for (int r : mine[w]) {
+        prk::RxRec o = rx0[slot_of[r]];
+        o.qoff = (r - r0) * 64;
+        rx.push_back(o);
+      }
+      rrange.push_back((int32_t)rx.size());
+    }
+    for (int k = 0; k < m->nsp; ++k) {
+      const int e0 = m->inc_start[k], e1 = m->inc_start[k + 1];
+      for (int b = e0; b < e1; b += PR_GATHER_BLOCK) {
+        const int be = std::min(e1, b + PR_GATHER_BLOCK);
+        prk::GatherPiece p{};
+        for (int e = b; e < be; ++e) {
+          if (m->inc_r[e] < r0 || m->inc_r[e] >= r1) continue;
+          if (p.ne == 0) p.first = e == b;
+          p.nu[p.ne] = (double)m->inc_nu[e];
+          p.qoff[p.ne++] = (m->inc_r[e] - r0) * 64;
+          p.last = e == be - 1;
+        }
+        p.lead = b == e0;
+        if (p.ne) pieces.push_back(p);
+      }
+      prange.push_back((int32_t)pieces.size());
+    }
+  }
+  std::vector<unsigned char> out;
+  auto put = [&](const void* p, size_t bytes) {
+    const size_t at = (out.size() + 63) / 64 * 64;
+    out.resize(at + bytes, 0);
+    std::memcpy(out.data() + at, p, bytes);
+    return at;
+  };
+  off[0] = put(rx.data(), sizeof(prk::RxRec) * rx.size());
+  off[1] = put(rrange.data(), sizeof(int32_t) * rrange.size());
+  off[2] = put(pieces.data(), sizeof(prk::GatherPiece) * pieces.size());
+  off[3] = put(prange.data(), sizeof(int32_t) * prange.size());
+  return out;
 }
 
 struct Keys {
@@ -426,6 +546,9 @@ struct pr_handle {
   int block = 128;
   unsigned char* d_blob = nullptr;
   int blob_bytes = 0;
+  const BlockOps* blk = nullptr;
+  prk::BlockTabs tabs{};       // device tables of the block kernels, one allocation
+  void* d_tabs = nullptr;
   double* d_atolv = nullptr;
   void* d_counters = nullptr;  // two regions of 128 B: queue (4 B), nfail (4 B), stats (8 x 8 B at +64)
   double* d_gscr = nullptr;    // per-group global scratch slots
@@ -513,8 +636,13 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
   }
   // per-component absolute tolerances: ode.atol everywhere until set_typ_vals_ode scales them
   // (the kernels always read this array, so a captured graph sees later typical values)
+  size_t toff[4];
+  h->blk = find_block_ops(m->name);
+  const std::vector<unsigned char> tabs = pack_block_tabs(m, blob, h->blk->waves, h->blk->nchunk, toff);
   const std::vector<double> atol0((size_t)m->nsp + 1, K.atol);
   if (hipMalloc(&h->d_blob, blob.size()) != hipSuccess || hipMalloc(&h->d_counters, 256) != hipSuccess ||
+      hipMalloc(&h->d_tabs, tabs.size()) != hipSuccess ||
+      hipMemcpy(h->d_tabs, tabs.data(), tabs.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMalloc(&h->d_atolv, sizeof(double) * (m->nsp + 1)) != hipSuccess ||
       hipMemcpy(h->d_atolv, atol0.data(), sizeof(double) * atol0.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(h->d_blob, blob.data(), blob.size(), hipMemcpyHostToDevice) != hipSuccess ||
@@ -522,6 +650,14 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
       hipEventCreate(&h->ev2) != hipSuccess || hipEventCreate(&h->ev3) != hipSuccess) {
     pr_destroy(h);
     return fail(PR_ERR_HIP, "device allocation failed");
+  }
+  {
+    auto* t = static_cast<unsigned char*>(h->d_tabs);
+    h->tabs.rx = reinterpret_cast<const prk::RxRec*>(t + toff[0]);
+    h->tabs.rx_range = reinterpret_cast<const int32_t*>(t + toff[1]);
+    h->tabs.piece = reinterpret_cast<const prk::GatherPiece*>(t + toff[2]);
+    h->tabs.piece_range = reinterpret_cast<const int32_t*>(t + toff[3]);
+    h->tabs.nchunk = h->blk->nchunk;
   }
   *out = h;
   return 0;
@@ -1620,16 +1756,25 @@ int pr_reaction_rate_box(pr_handle* h, const int lo[3], const int hi[3], const p
   P.blob_bytes = h->blob_bytes;
   P.neff = h->mech->neff;
   P.ninc = h->mech->ninc;
-  const int G = h->var->G;
-  const int block = pick_block(h);
-  const size_t shmem = (size_t)h->blob_bytes + (size_t)(block / G) * h->var->scratch;
   int dev_cus = 0;
   HIPCHK(hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, h->device));
-  const long want = (ncells + (block / G) - 1) / (block / G);
-  const long cap = 8L * dev_cus;
-  const int blocks = (int)(want < cap ? want : cap);
   hipStream_t st = (hipStream_t)stream;
-  HIPCHK(h->var->rate(P, blocks, block, shmem, st));
+  // One cell per lane (64 cells per block, rates_block_kernel) once the box keeps the CUs busy that
+  // way; below, a group of lanes per cell, which spreads few cells over more wavefronts. Measured
+  // (us per call, groups / blocks): drm19 4096 cells 32 / 51, 13824 51 / 52, 32768 86 / 57, 262144
+  // 471 / 222; LiDryer 4096 28 / 31, 13824 34 / 31, 110592 95 / 51; dodecane_lu 1728 44 / 71, 4096
+  // 61 / 71, 13824 125 / 73, 110592 747 / 367. The crossing is near 48 cells per CU up to 32
+  // components and 24 above.
+  if (ncells >= (N + 1 <= 32 ? 48L : 24L) * dev_cus) {
+    HIPCHK(h->blk->rates(P, h->tabs, dev_cus, st));
+  } else {
+    const int G = h->var->G;
+    const int block = pick_block(h);
+    const size_t shmem = (size_t)h->blob_bytes + (size_t)(block / G) * h->var->scratch;
+    const long want = (ncells + (block / G) - 1) / (block / G);
+    const long cap = 8L * dev_cus;
+    HIPCHK(h->var->rate(P, (int)(want < cap ? want : cap), block, shmem, st));
+  }
   HIPCHK(hipStreamSynchronize(st));
   return 0;
 }
@@ -2209,6 +2354,7 @@ void pr_destroy(pr_handle* h) {
   if (!h) return;
   if (h->d_blob) (void)hipFree(h->d_blob);
   if (h->d_counters) (void)hipFree(h->d_counters);
+  if (h->d_tabs) (void)hipFree(h->d_tabs);
   if (h->d_atolv) (void)hipFree(h->d_atolv);
   if (h->d_gscr) (void)hipFree(h->d_gscr);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
