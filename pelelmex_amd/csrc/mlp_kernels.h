@@ -44,74 +44,148 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
   return cdf + z * pdf;
 }
 
-// Block tile 64 x 64, K step 32, 256 threads = 4 waves in a 2 x 2 arrangement of 32 x 32 wave
-// tiles, each wave tile = 2 x 2 MFMA 16 x 16 x 32 tiles. Operand tiles are staged in LDS with k
-// fastest (row pitch 40 bf16 = 80 bytes, so the 16-byte operand reads of neighbouring rows fall
-// in different banks). MFMA lane layout: lane l supplies A row l % 16 and B column l % 16 with
-// k = 8 (l / 16) .. 8 (l / 16) + 7, and receives D rows 4 (l / 16) .. + 3 of column l % 16.
-constexpr int GT_M = 64, GT_N = 64, GT_K = 32, G_PITCH = 40;
+// Products with operands in any layout. A wave forms a 32 x 32 tile as 2 x 2 MFMA 16 x 16 x 32
+// tiles, its operands going from memory straight into the MFMA registers: the matrices are small
+// (they sit in L2) and a K step's loads are issued one step ahead, so staging through LDS would
+// only add two barriers a step. MFMA lane layout: lane l supplies A row l % 16 and B column l % 16
+// with k = 8 (l / 16) .. 8 (l / 16) + 7, and receives D rows 4 (l / 16) .. + 3 of column l % 16.
+// How an operand is read (x: its row m or column n):
+//   LD_K     k contiguous, 16-byte aligned rows: one 16-byte load per tile
+//   LD_PAIR  x contiguous, 4-byte aligned, even extent: one 4-byte load per k gives rows 2 r and
+//            2 r + 1, which go to the wave's two tiles (tile i holds rows 2 r + i)
+//   LD_ANY   any strides: one 2-byte load per element
+// Blocks: KS == 1: 4 waves cover 64 x 64 (2 x 2), each over the whole K. KS > 1: KS waves share one
+// 32 x 32 tile, wave w taking the K steps w, w + KS, ..; their partial tiles are added in wave order
+// through LDS. The split is for products with a long K and a small result (weight gradients: K is
+// the batch, 16 tiles of 64 x 64 for a 256 x 256 layer on 256 CUs). What bounds both is the latency
+// of the loads, not the matrix cores. Products of a
+// training step (batch 4096, 4 layers of 256), 14 in all: 2790 us with operands staged element by
+// element through LDS and no split, 188 us now (a weight gradient 530 -> 16, a forward layer 36 ->
+// 16, a data gradient 25 -> 9).
+constexpr int GT_K = 32, G_PITCH = 40;
+enum { LD_K = 0, LD_PAIR = 1, LD_ANY = 2 };
+constexpr int kSplitWaves = 16;
 
-__global__ void __launch_bounds__(256) gemm_bf16_kernel(GemmParams P) {
-  __shared__ __align__(16) __bf16 As[GT_M * G_PITCH];
-  __shared__ __align__(16) __bf16 Bs[GT_N * G_PITCH];
-  const int t = threadIdx.x;
-  const int wave = t / 64, l = t % 64;
-  const int m0 = blockIdx.y * GT_M, n0 = blockIdx.x * GT_N;
-  const int wm = (wave / 2) * 32, wn = (wave % 2) * 32;
+// Fragments of the wave's two tiles from operand X (element (x, k) at p[x * sx + k * sk]), rows
+// x0 .. x0 + 31, k0 .. k0 + 31. Rows past nx read row nx - 1 (their results are not stored), k past
+// K is zero in both operands.
+template <int LD>
+__device__ __forceinline__ void load_frags(const __bf16* __restrict__ p, long sx, long sk, int x0, int nx, int k0,
+                                           int K, int l, bf16x8 (&f)[2]) {
+  const int r = l % 16, k = k0 + 8 * (l / 16);
+  const __bf16 zero = (__bf16)0.0f;
+  if constexpr (LD == LD_K) {  // K is a multiple of 8: a chunk of 8 is inside or outside
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = x0 + 16 * i + r;
+      f[i] = *reinterpret_cast<const bf16x8*>(p + (long)(x < nx ? x : nx - 1) * sx + (k < K ? k : 0));
+    }
+    if (k >= K)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[0][j] = f[1][j] = zero;
+  } else if constexpr (LD == LD_PAIR) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const int x = x0 + 2 * r;
+    const __bf16* q = p + (x < nx ? x : nx - 2);
+    bf16x2 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const bf16x2*>(q + (long)(k + j < K ? k + j : 0) * sk);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      f[0][j] = k + j < K ? v[j][0] : zero;
+      f[1][j] = k + j < K ? v[j][1] : zero;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = x0 + 16 * i + r;
+      const __bf16* q = p + (long)(x < nx ? x : nx - 1) * sx;
+      __bf16 v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = q[(long)(k + j < K ? k + j : 0) * sk];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[i][j] = k + j < K ? v[j] : zero;
+    }
+  }
+}
+
+// Row (or column) of the operand that tile i's row r holds.
+template <int LD>
+__device__ __forceinline__ int frag_row(int i, int r) {
+  return LD == LD_PAIR ? 2 * r + i : 16 * i + r;
+}
+
+__device__ __forceinline__ void gemm_store(const GemmParams& P, int gm, int gn, float v) {
+  if (gm >= P.M || gn >= P.N) return;
+  if (P.accumulate) {
+    P.C[(long)gm * P.ldc + gn] += v;
+    return;
+  }
+  if (P.bias) v += P.bias[gn];
+  if (P.Z) P.Z[(long)gm * P.ldz + gn] = v;
+  if (P.epi == EPI_GELU) v = gelu_f(v);
+  if (P.C) P.C[(long)gm * P.ldc + gn] = v;
+  if (P.Cb) P.Cb[(long)gm * P.ldcb + gn] = (__bf16)v;
+}
+
+template <int LA, int LB, int KS>
+__global__ void __launch_bounds__(KS == 1 ? 256 : 64 * KS) gemm_bf16_kernel(GemmParams P) {
+  const int wave = threadIdx.x / 64, l = threadIdx.x % 64;
+  const int m0 = KS == 1 ? blockIdx.y * 64 + (wave / 2) * 32 : blockIdx.y * 32;
+  const int n0 = KS == 1 ? blockIdx.x * 64 + (wave % 2) * 32 : blockIdx.x * 32;
+  if (KS == 1 && (m0 >= P.M || n0 >= P.N)) return;  // no barrier on this path
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bool a_kfast = (P.sak == 1), b_kfast = (P.sbk == 1);
-  for (int k0 = 0; k0 < P.K; k0 += GT_K) {
-    // stage: 2048 elements per operand tile, 8 per thread, consecutive threads on the
-    // operand's contiguous dimension
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int e = t + 256 * j;
-      int m, k;
-      if (a_kfast) { m = e / GT_K; k = e % GT_K; } else { k = e / GT_M; m = e % GT_M; }
-      const int gm = m0 + m, gk = k0 + k;
-      As[m * G_PITCH + k] = (gm < P.M && gk < P.K) ? P.A[(long)gm * P.sam + (long)gk * P.sak] : (__bf16)0.0f;
-      int n;
-      if (b_kfast) { n = e / GT_K; k = e % GT_K; } else { k = e / GT_N; n = e % GT_N; }
-      const int gn = n0 + n;
-      const int gk2 = k0 + k;
-      Bs[n * G_PITCH + k] = (gn < P.N && gk2 < P.K) ? P.B[(long)gk2 * P.sbk + (long)gn * P.sbn] : (__bf16)0.0f;
-    }
-    __syncthreads();
-    bf16x8 a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(&As[(wm + 16 * i + l % 16) * G_PITCH + 8 * (l / 16)]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const bf16x8*>(&Bs[(wn + 16 * j + l % 16) * G_PITCH + 8 * (l / 16)]);
+  const int step = GT_K * KS;
+  int k0 = KS == 1 ? 0 : GT_K * wave;
+  bf16x8 a[2], b[2];
+  if (k0 < P.K) {
+    load_frags<LA>(P.A, P.sam, P.sak, m0, P.M, k0, P.K, l, a);
+    load_frags<LB>(P.B, P.sbn, P.sbk, n0, P.N, k0, P.K, l, b);
+  }
+  for (; k0 < P.K; k0 += step) {
+    bf16x8 an[2], bn[2];  // the next step's operands (past the end: zeros, not used)
+    load_frags<LA>(P.A, P.sam, P.sak, m0, P.M, k0 + step, P.K, l, an);
+    load_frags<LB>(P.B, P.sbn, P.sbk, n0, P.N, k0 + step, P.K, l, bn);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      a[i] = an[i];
+      b[i] = bn[i];
+    }
   }
+  if constexpr (KS == 1) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gm = m0 + wm + 16 * i + 4 * (l / 16) + r;
-        const int gn = n0 + wn + 16 * j + l % 16;
-        if (gm >= P.M || gn >= P.N) continue;
-        float v = acc[i][j][r];
-        if (P.accumulate) {
-          P.C[(long)gm * P.ldc + gn] += v;
-          continue;
-        }
-        if (P.bias) v += P.bias[gn];
-        if (P.Z) P.Z[(long)gm * P.ldz + gn] = v;
-        if (P.epi == EPI_GELU) v = gelu_f(v);
-        if (P.C) P.C[(long)gm * P.ldc + gn] = v;
-        if (P.Cb) P.Cb[(long)gm * P.ldcb + gn] = (__bf16)v;
-      }
+        for (int r = 0; r < 4; ++r)
+          gemm_store(P, m0 + frag_row<LA>(i, 4 * (l / 16) + r), n0 + frag_row<LB>(j, l % 16), acc[i][j][r]);
+  } else {
+    __shared__ float part[KS][32 * 33];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          part[wave][frag_row<LA>(i, 4 * (l / 16) + r) * 33 + frag_row<LB>(j, l % 16)] = acc[i][j][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 1024; e += 64 * KS) {
+      const int m = e / 32, n = e % 32;
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < KS; ++w) v += part[w][m * 33 + n];
+      gemm_store(P, m0 + m, n0 + n, v);
+    }
+  }
 }
 
 // Forward product of a hidden layer on the inference path: A [M x K] row-major (k fastest, lda =
@@ -216,21 +290,28 @@ __global__ void gelu_bwd_kernel(long rows, int cols, const float* dA, long lda, 
   if (dZ) dZ[r * ldd + c] = g;
 }
 
-// db[c] = sum over rows of d[r, c] (one block per 64 columns, rows strided over the block).
-__global__ void __launch_bounds__(256) col_sum_kernel(long rows, int cols, const float* d, long ld, float* out,
-                                                      int accumulate) {
-  __shared__ float part[4][64];
-  const int c = blockIdx.x * 64 + threadIdx.x % 64;
-  const int rg = threadIdx.x / 64;
+// db[c] = sum over rows of d[r, c]: 16 columns per block, 64 row groups of 16 lanes, each summing
+// its rows (r, r + 64, ..) with eight loads in flight, then a pairwise tree over the groups. 16
+// columns and not 64 per block: a layer of 256 then has 16 blocks instead of 4 (4096 rows: 240 us
+// with 4 row groups and 64 columns, 9 us now).
+constexpr int kSumCols = 16;
+__global__ void __launch_bounds__(1024) col_sum_kernel(long rows, int cols, const float* d, long ld, float* out,
+                                                       int accumulate) {
+  __shared__ float part[64][kSumCols];
+  const int cl = threadIdx.x % kSumCols, rg = threadIdx.x / kSumCols;
+  const int c = blockIdx.x * kSumCols + cl;
   float s = 0.f;
-  if (c < cols)
-    for (long r = rg; r < rows; r += 4) s += d[r * ld + c];
-  part[rg][threadIdx.x % 64] = s;
-  __syncthreads();
-  if (rg == 0 && c < cols) {
-    const float v = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
-    out[c] = accumulate ? out[c] + v : v;
+  if (c < cols) {
+#pragma unroll 8
+    for (long r = rg; r < rows; r += 64) s += d[r * ld + c];
   }
+  part[rg][cl] = s;
+  __syncthreads();
+  for (int w = 32; w > 0; w >>= 1) {
+    if (rg < w) part[rg][cl] += part[rg + w][cl];
+    __syncthreads();
+  }
+  if (rg == 0 && c < cols) out[c] = accumulate ? out[c] + part[0][cl] : part[0][cl];
 }
 
 // Mean-squared error over the first `cols` outputs: dY = 2 (Y - T) / (rows cols) (fp32, row

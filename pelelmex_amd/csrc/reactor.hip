@@ -150,6 +150,30 @@ constexpr int scratch_bytes() {
   return prk::group_doubles<N, R, G>() * 8;
 }
 
+// How gemm_bf16_kernel reads an operand of nx rows (element (x, k) at p[x * sx + k * sk]).
+int gemm_ld(const __bf16* p, long sx, long sk, int nx, int K) {
+  const auto at = reinterpret_cast<uintptr_t>(p);
+  if (sk == 1 && sx % 8 == 0 && K % 8 == 0 && at % 16 == 0) return prk::LD_K;
+  if (sx == 1 && sk % 2 == 0 && nx % 2 == 0 && at % 4 == 0) return prk::LD_PAIR;
+  return prk::LD_ANY;
+}
+
+template <int LA, int LB>
+hipError_t gemm_launch_t(const prk::GemmParams& G, hipStream_t st) {
+  // K split over the waves of a block: only where K is the longest side, and only for bare
+  // products (gradients), so that a forward product keeps one order of summation at every batch
+  // size. Below 256 a block's waves would have no step each.
+  const bool bare = !G.bias && G.epi == prk::EPI_NONE && !G.Cb && !G.Z;
+  if (bare && G.K > G.M && G.K > G.N && G.K >= 256 && G.M <= 65535 * 32) {
+    const dim3 grid((unsigned)((G.N + 31) / 32), (unsigned)((G.M + 31) / 32));
+    hipLaunchKernelGGL((prk::gemm_bf16_kernel<LA, LB, prk::kSplitWaves>), grid, dim3(64 * prk::kSplitWaves), 0, st, G);
+  } else {
+    const dim3 grid((unsigned)((G.N + 63) / 64), (unsigned)((G.M + 63) / 64));
+    hipLaunchKernelGGL((prk::gemm_bf16_kernel<LA, LB, 1>), grid, dim3(256), 0, st, G);
+  }
+  return hipGetLastError();
+}
+
 struct Variant {
   const char* mech;
   int G;
@@ -865,9 +889,18 @@ static int ensure_surr_buffers(pr_handle* h, long ncells) {
 
 static hipError_t gemm_launch(const prk::GemmParams& G, hipStream_t st) {
   if (G.M <= 0 || G.N <= 0) return hipSuccess;
-  dim3 grid((unsigned)((G.N + prk::GT_N - 1) / prk::GT_N), (unsigned)((G.M + prk::GT_M - 1) / prk::GT_M));
-  hipLaunchKernelGGL(prk::gemm_bf16_kernel, grid, dim3(256), 0, st, G);
-  return hipGetLastError();
+  const int la = gemm_ld(G.A, G.sam, G.sak, G.M, G.K), lb = gemm_ld(G.B, G.sbn, G.sbk, G.N, G.K);
+  switch (3 * la + lb) {
+    case 3 * prk::LD_K + prk::LD_K: return gemm_launch_t<prk::LD_K, prk::LD_K>(G, st);
+    case 3 * prk::LD_K + prk::LD_PAIR: return gemm_launch_t<prk::LD_K, prk::LD_PAIR>(G, st);
+    case 3 * prk::LD_K + prk::LD_ANY: return gemm_launch_t<prk::LD_K, prk::LD_ANY>(G, st);
+    case 3 * prk::LD_PAIR + prk::LD_K: return gemm_launch_t<prk::LD_PAIR, prk::LD_K>(G, st);
+    case 3 * prk::LD_PAIR + prk::LD_PAIR: return gemm_launch_t<prk::LD_PAIR, prk::LD_PAIR>(G, st);
+    case 3 * prk::LD_PAIR + prk::LD_ANY: return gemm_launch_t<prk::LD_PAIR, prk::LD_ANY>(G, st);
+    case 3 * prk::LD_ANY + prk::LD_K: return gemm_launch_t<prk::LD_ANY, prk::LD_K>(G, st);
+    case 3 * prk::LD_ANY + prk::LD_PAIR: return gemm_launch_t<prk::LD_ANY, prk::LD_PAIR>(G, st);
+    default: return gemm_launch_t<prk::LD_ANY, prk::LD_ANY>(G, st);
+  }
 }
 
 // Network forward over feature rows [r0, r0 + m) of S->X: hidden layers GELU into bf16, last
@@ -2307,7 +2340,7 @@ int pr_mlp_gelu_backward(int64_t rows, int cols, const float* dA, int64_t lda, c
 
 int pr_mlp_column_sum(int64_t rows, int cols, const float* d, int64_t ld, float* out, int accumulate, void* stream) {
   if (rows < 0 || cols < 1 || !d || !out) return fail(PR_ERR_ARG, "bad argument");
-  hipLaunchKernelGGL(prk::col_sum_kernel, dim3((unsigned)((cols + 63) / 64)), dim3(256), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL(prk::col_sum_kernel, dim3((unsigned)((cols + prk::kSumCols - 1) / prk::kSumCols)), dim3(1024), 0, (hipStream_t)stream,
                      (long)rows, cols, d, (long)ld, out, accumulate);
   HIPCHK(hipGetLastError());
   return 0;

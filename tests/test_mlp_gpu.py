@@ -135,3 +135,44 @@ def test_hidden_layer_forward_kernel_bits(gpu):
     assert torch.isfinite(Y1).all()
     assert torch.equal(Y1, Y2)
     r.close()
+
+
+# gradients' products: K split over a block's waves from 256 on when it is the longest side; the
+# smallest split, ragged tiles and K steps, odd extents and strides, both sides of 64 x 64
+@pytest.mark.parametrize("a_kfast,b_kfast", [(True, False), (True, True), (False, False), (False, True)])
+@pytest.mark.parametrize("M,N,K", [(255, 33, 256), (23, 256, 4096), (256, 22, 1031), (1, 1, 511), (34, 66, 520)])
+def test_gemm_long_k(gpu, a_kfast, b_kfast, M, N, K):
+    import torch
+    from pelelmex_amd import surrogate as sg
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+    Ab, Bb = mo.bf16_round(A), mo.bf16_round(B)
+    Ad = (_bf16(A) if a_kfast else _bf16(A.T.copy())).to(gpu).contiguous()
+    Bd = (_bf16(B.T.copy()) if b_kfast else _bf16(B)).to(gpu).contiguous()
+    sam, sak = (K, 1) if a_kfast else (1, M)
+    sbk, sbn = (1, K) if b_kfast else (N, 1)
+    # fp32 additions of one element: 32 inside an MFMA, one per K step of a wave, one per wave; each
+    # may be off by 2^-23 of the running sum, which the sum of magnitudes bounds
+    tol = (32 + K / 512 + 1 + 16) * 2.0 ** -23 * (np.abs(Ab) @ np.abs(Bb))
+    for off in (0, 1):  # the second pass from an odd element, so that no wide load is aligned
+        Ao = torch.cat([Ad.flatten()[:off], Ad.flatten()])[off:]
+        Bo = torch.cat([Bd.flatten()[:off], Bd.flatten()])[off:]
+        C = torch.full((M, N), float("nan"), dtype=torch.float32, device=gpu)
+        sg.gemm(M, N, K, Ao, sam, sak, Bo, sbk, sbn, Cf=C, ldc=N)
+        torch.cuda.synchronize()
+        assert np.all(np.abs(C.cpu().numpy() - Ab @ Bb) <= tol)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (63, 15), (64, 16), (65, 17), (4097, 22), (600, 256)])
+def test_column_sum(gpu, rows, cols):
+    import torch
+    from pelelmex_amd import surrogate as sg
+    from pelelmex_amd.reactor import lib
+    d = torch.randn((rows, cols + 3), generator=torch.Generator().manual_seed(rows)).to(gpu)
+    out = torch.full((cols,), 2.0, dtype=torch.float32, device=gpu)
+    ref = d[:, :cols].double().sum(0)
+    tol = (rows / 64 + 7) * 2.0 ** -23 * d[:, :cols].double().abs().sum(0)
+    for acc, base in ((0, 0.0), (1, ref)):
+        assert lib().pr_mlp_column_sum(rows, cols, sg._ptr(d), cols + 3, sg._ptr(out), acc, sg._stream()) == 0
+        torch.cuda.synchronize()
+        assert torch.all((out.double() - base - ref).abs() <= (1 + 2 * acc) * tol + acc * 2.0 ** -22 * ref.abs())
