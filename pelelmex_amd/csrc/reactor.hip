@@ -247,6 +247,27 @@ const Variant* find_variant(const char* mech, int G, int W = 0) {
   return nullptr;
 }
 
+// Small launches: the launch lasts as long as its stiffest cell's integration (four times the mean's
+// right-hand sides) whatever is idle, so a cell gets more lanes (fewer passes over the reactions) and
+// shares its wavefront with fewer others (no waiting for their Jacobians and factorizations). A rule
+// holds for launches of up to max_cells cells when no key chooses a variant; all variants give the
+// same bits. The lines lie where the wider variant stops winning when cells come in natural order (a
+// first call); with the cost order they would lie higher. Measured, ms per call, natural order /
+// cost order: drm19, 64 lanes against 32: 512 cells 7.1 / 7.2 against 11.8 / 10.9, 4096 9.5 / 7.9
+// against 11.8 / 11.7, 5832 11.5 / 7.7 against 12.5 / 11.9, 8000 13.8 / 8.1 against 13.1 / 12.5.
+// LiDryer, 64 / 32 / 16 lanes: 512 cells 1.63 / 1.74 / 2.85 natural, 1.63 / 1.78 / 2.28 ordered;
+// 1728 1.91 / 1.85 / 2.79 and 1.70 / 1.92 / 2.4; 5832 3.81 / 2.40 / 2.93 natural; 8000 4.8 / 3.0 /
+// 2.97 and 4.0 / 2.2 / 2.65. 54 components run 64 lanes at every size.
+struct SizeRule {
+  long max_cells;
+  Variant v;
+};
+const SizeRule kSizeRules[] = {  // per mechanism in ascending order
+    {2048, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 64, 2)},
+    {7168, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 32, 3)},
+    {6144, PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 64, 2)},
+};
+
 std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
   prk::BlobLayout L = prk::blob_layout(m->nsp, m->nr, m->neff, m->ninc);
   std::vector<unsigned char> b(L.bytes, 0);
@@ -724,18 +745,32 @@ static int pick_block(const pr_handle* h) {
 // Block size of the BDF kernel: hipbdf.block when set, else the largest block (up to
 // 256 * waves threads) whose LDS (mechanism tables + per-group areas) lets the variant's waves
 // per SIMD be resident, i.e. ceil(256 * waves / b) blocks per CU.
-static int bdf_block(const pr_handle* h) {
+static int bdf_block(const pr_handle* h, const Variant* v) {
   if (h->block) return h->block;
-  const int G = h->var->G, W = h->var->waves;
+  const int G = v->G, W = v->waves;
   for (int b = 256 * W; b >= 64; b -= 64) {
     const size_t per_cu = (size_t)((256 * W + b - 1) / b);
-    if ((size_t)h->blob_bytes + (size_t)(b / G) * h->var->scratch <= kLdsPerCU / per_cu) return b;
+    if ((size_t)h->blob_bytes + (size_t)(b / G) * v->scratch <= kLdsPerCU / per_cu) return b;
   }
   return 64;
 }
 
-static int ensure_gscr(pr_handle* h, long slots) {
-  const size_t need = (size_t)slots * (size_t)h->var->slot;
+// BDF kernel of a launch of up to work cells: the handle's variant, unless the keys leave the
+// choice open and the launch is small (kSizeRules). All variants give the same bits.
+static const Variant* bdf_variant(const pr_handle* h, long work, int* block) {
+  const Keys& K = h->keys;
+  const Variant* v = h->var;
+  if (!K.lanes_per_cell && !K.waves && !K.block && !K.autotune)
+    for (const SizeRule& r : kSizeRules)
+      if (std::strcmp(r.v.mech, h->mech->name) == 0 && work <= r.max_cells) {
+        v = &r.v;
+        break;
+      }
+  *block = bdf_block(h, v);
+  return v;
+}
+
+static int ensure_gscr(pr_handle* h, size_t need) {
   if (need <= h->gscr_bytes) return 0;
   release(h, h->d_gscr);
   h->d_gscr = nullptr;
@@ -765,19 +800,21 @@ static prk::Arr to_arr(const pr_array4* a) {
 // bytes and the grid is capped to the groups it holds; otherwise the handle's slots grow to fit.
 static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t st, double* gscr = nullptr,
                       size_t gscr_cap = 0) {
-  const int G = h->var->G;
-  const int block = bdf_block(h);
-  if (block > 256 * h->var->waves)
-    return fail(PR_ERR_KEY, "hipbdf.block " + std::to_string(block) + " exceeds " + std::to_string(256 * h->var->waves) +
+  int block = 0;
+  const Variant* v = bdf_variant(h, work_max, &block);
+  const int G = v->G;
+  if (block > 256 * v->waves)
+    return fail(PR_ERR_KEY, "hipbdf.block " + std::to_string(block) + " exceeds " + std::to_string(256 * v->waves) +
                                 " threads for " + std::to_string(G) + " lanes per cell");
-  const size_t shmem = (size_t)h->blob_bytes + (size_t)(block / G) * h->var->scratch;
+  const size_t shmem = (size_t)h->blob_bytes + (size_t)(block / G) * v->scratch;
   int dev_cus = 0, nb = 0;
   HIPCHK(hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, h->device));
-  HIPCHK(h->var->occ(&nb, block, shmem));
+  HIPCHK(v->occ(&nb, block, shmem));
   if (nb < 1) return fail(PR_ERR_HIP, "kernel does not fit on a CU with this block / LDS size");
   long cap = (long)nb * dev_cus;
   if (gscr) {
-    const long fit = (long)(gscr_cap / ((size_t)(block / G) * (size_t)h->var->slot));
+    const size_t per = (size_t)(block / G) * (size_t)v->slot;  // 0: a variant without global slots
+    const long fit = per ? (long)(gscr_cap / per) : cap;
     if (fit < 1) return fail(PR_ERR_ARG, "scratch too small for one block of this kernel variant");
     cap = fit < cap ? fit : cap;
   }
@@ -787,17 +824,24 @@ static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t 
   if (gscr) {
     P.gscr = gscr;
   } else {
-    int rc = ensure_gscr(h, (long)blocks * (block / G));
+    size_t need = (size_t)blocks * (size_t)(block / G) * (size_t)v->slot;
+    // a smaller launch of this handle may take another variant; it finds its slots allocated, as a
+    // captured one has to
+    if (v == h->var)
+      for (const SizeRule& r : kSizeRules)
+        if (std::strcmp(r.v.mech, h->mech->name) == 0)
+          need = std::max(need, (size_t)(r.max_cells + 256 * r.v.waves / r.v.G) * (size_t)r.v.slot);
+    int rc = ensure_gscr(h, need);
     if (rc) return rc;
     P.gscr = h->d_gscr;
   }
   hipLaunchKernelGGL(prk::zero_counters, dim3(1), dim3(64), 0, st, P.queue, P.stats, P.nfail);
   HIPCHK(hipGetLastError());
-  HIPCHK(h->var->launch(P, blocks, block, shmem, st));
+  HIPCHK(v->launch(P, blocks, block, shmem, st));
   h->last.lanes_per_cell = G;
   h->last.blocks = blocks;
   h->last.block_threads = block;
-  h->last.waves_per_simd = h->var->waves;
+  h->last.waves_per_simd = v->waves;
   return 0;
 }
 
@@ -1010,7 +1054,7 @@ static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc&
     for (int blk : {0, 256, 128}) {  // 0: the variant's own choice (bdf_block)
       h->var = &v;
       h->block = 0;
-      if (blk != 0 && blk == bdf_block(h)) continue;
+      if (blk != 0 && blk == bdf_block(h, h->var)) continue;
       h->block = blk;
       prk::KParams P = Pbase;
       const prk::BoxDesc* db = nullptr;
@@ -1731,7 +1775,7 @@ static int eval_batch(pr_handle* h, int mode, int64_t ncells, const double* y, c
   const long cap = (long)nb * dev_cus;
   const int blocks = (int)(want < cap ? want : cap);
   {
-    int rc = ensure_gscr(h, (long)blocks * (block / G));
+    int rc = ensure_gscr(h, (size_t)blocks * (size_t)(block / G) * (size_t)h->var->slot);
     if (rc) return rc;
   }
   hipStream_t st = (hipStream_t)stream;

@@ -1,5 +1,6 @@
-"""The kernels that take 64 cells per block (csrc/block_rates.h), against the CPU oracle bit for
-bit at the sizes where their dispatch and their last block change."""
+"""Launches whose kernel depends on the number of cells, at the sizes where it changes: the kernels
+that take 64 cells per block (csrc/block_rates.h) against the CPU oracle bit for bit, and the BDF's
+variants for small launches against the one of large launches."""
 import numpy as np
 import pytest
 
@@ -47,3 +48,26 @@ def test_reaction_rates_64_cells_per_block(gpu, mech, dims):
                          mask=dev(mask, nz, ny, nx), rYdot=out)
     r.close()
     _bits("rYdot", out.cpu().numpy().reshape(m.nsp, nc), ref)
+
+
+@pytest.mark.parametrize("mech,cells,lanes", [("LiDryer", 1, 64), ("LiDryer", 2048, 64), ("LiDryer", 2049, 32),
+                                              ("LiDryer", 7168, 32), ("LiDryer", 7169, 16), ("drm19", 1, 64),
+                                              ("drm19", 6144, 64), ("drm19", 6145, 32)])
+def test_react_variant_by_size(gpu, mech, cells, lanes):
+    """A launch's variant follows its cell count unless a key chooses one; the bits do not."""
+    import torch
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    box = BOXES[mech](nx=cells, ny=1, nz=1)
+    out = []
+    for keys in (KEYS, dict(KEYS, **{"hipbdf.lanes_per_cell": 16 if mech == "LiDryer" else 32})):
+        r = Reactor.create("ReactorCvode", mech, dict(keys, **{"cvode.max_order": 4}))
+        r.init(2, 1)
+        t = box_tensors(box, gpu)
+        nfail, _, _ = r.react(t["rY"], t["rYsrc"], t["T"], t["rH"], t["rHsrc"], t["FC"], t["mask"], box["dt"], 0.0)
+        torch.cuda.synchronize()
+        out.append([t[k].cpu().numpy() for k in ("rY", "T", "rH", "FC")] + [nfail, r.stats()])
+        r.close()
+    assert out[0][5]["lanes_per_cell"] == lanes
+    for k in range(4):
+        _bits(("rY", "T", "rH", "FC")[k], out[0][k], out[1][k])
+    assert out[0][4] == out[1][4] and all(out[0][5][k] == out[1][5][k] for k in ("nst", "nfe", "nje", "nsetups", "nni"))
