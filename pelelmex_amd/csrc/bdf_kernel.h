@@ -59,6 +59,27 @@ struct BoxDesc {
   const double* dtv;  // per-cell dt_react (linear box index), nullable: dt for every cell
 };
 
+// Entry (k, j) of the species block, and of each species' sums over its reactions, as an ordered
+// list of terms ((coef rec[rec]) c1) c2: the incidence list of species k, restricted to what enters
+// column j. Entries are sorted by length and stored in slices of 64: term i of the slice's entry l
+// is at slice + 64 i + l, so neighbouring lanes read neighbouring terms at every group width.
+struct __align__(16) JacTerm {
+  double coef;      // nu (kf terms, rate and dq/dT sums), -nu (kr terms), nu times an efficiency
+  int32_t rec;      // double offset in the records [5][R]
+  uint16_t c1, c2;  // byte offsets from the concentrations; 48 N holds 1.0
+};
+struct JacEntry {
+  int32_t nt;   // number of terms
+  int32_t dst;  // k n + j, or ~(double offset from the concentrations) of a species' sum
+};
+struct JacTabs {
+  const JacTerm* term;
+  const JacEntry* entry;  // padded to whole slices (dst: kJacNone)
+  const int32_t* slice;   // first term of each slice
+  int nentry;
+};
+constexpr int32_t kJacNone = -(1 << 30);
+
 struct KParams {
   BoxDesc one;           // host side: the box of a single-box call (staged into boxes[0])
   const BoxDesc* boxes;  // device table of the launch's boxes: queue entry q is cell
@@ -74,6 +95,7 @@ struct KParams {
   unsigned long long* stats;     // cells, nst, nfe, nje, nsetups, nni, netf, ncfn
   unsigned int* nfail;
   double* gscr;                  // per-group global scratch slots (saved Jacobian, Jacobian records)
+  JacTabs jt;
   int clean;                     // ode.clean_init_massfrac: integrate from max(rhoY, 0), add the rest back
   const int* cell_list;          // when set: queue entry q integrates box cell cell_list[q]
   const unsigned int* ncells_dev;  // when set: min(*ncells_dev, ncells) entries are integrated
@@ -154,6 +176,115 @@ __device__ __forceinline__ double pr_log(double x) {
 
 __device__ __forceinline__ double pr_log10(double x) { return pr_log(x) * PRK_INV_LN10; }
 __device__ __forceinline__ double pr_pow(double x, double y) { return pr_exp(y * pr_log(x)); }
+
+// pr_exp's constants, held in scalar registers over a loop: each polynomial step is then one
+// v_fma_f64 with a scalar addend and nothing else.
+struct ExpK {
+  double l2e, hi, lo, c13, c12, c11, c10, c9, c8, c7, c6, c5, c4, c3;
+};
+__device__ __forceinline__ ExpK exp_constants() {
+  return ExpK{kc(PRK_LOG2E),        kc(PRK_LN2_HI),       kc(PRK_LN2_LO),      kc(1.0 / 6227020800.0), kc(1.0 / 479001600.0),
+              kc(1.0 / 39916800.0), kc(1.0 / 3628800.0),  kc(1.0 / 362880.0),  kc(1.0 / 40320.0),      kc(1.0 / 5040.0),
+              kc(1.0 / 720.0),      kc(1.0 / 120.0),      kc(1.0 / 24.0),      kc(1.0 / 6.0)};
+}
+
+// M exponentials at once, the bits of pr_exp: M independent chains in one basic block (one chain of
+// 20 dependent FP64 operations leaves most issue slots of a wavefront empty). pr_exp's range tests
+// are one comparison per argument and a branch no wavefront takes in practice.
+template <int M>
+__device__ __forceinline__ void exp_n(const ExpK& K, const double (&x)[M], double (&e)[M]) {
+  bool far = false;
+#pragma unroll
+  for (int m = 0; m < M; ++m) far |= !(fabs(x[m]) < 700.0);
+  double k[M], r[M], p[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) k[m] = rint(x[m] * K.l2e);
+#pragma unroll
+  for (int m = 0; m < M; ++m) r[m] = fma(-k[m], K.hi, x[m]);
+#pragma unroll
+  for (int m = 0; m < M; ++m) r[m] = fma(-k[m], K.lo, r[m]);
+#pragma unroll
+  for (int m = 0; m < M; ++m) p[m] = fma(K.c13, r[m], K.c12);
+#define PRK_EXP_STEP(C) \
+  _Pragma("unroll") for (int m = 0; m < M; ++m) p[m] = fma(p[m], r[m], C)
+  PRK_EXP_STEP(K.c11);
+  PRK_EXP_STEP(K.c10);
+  PRK_EXP_STEP(K.c9);
+  PRK_EXP_STEP(K.c8);
+  PRK_EXP_STEP(K.c7);
+  PRK_EXP_STEP(K.c6);
+  PRK_EXP_STEP(K.c5);
+  PRK_EXP_STEP(K.c4);
+  PRK_EXP_STEP(K.c3);
+  PRK_EXP_STEP(0.5);
+  PRK_EXP_STEP(1.0);
+  PRK_EXP_STEP(1.0);
+#undef PRK_EXP_STEP
+#pragma unroll
+  for (int m = 0; m < M; ++m) e[m] = ldexp(p[m], (int)k[m]);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      if (x[m] > 709.782712893384) e[m] = __builtin_huge_val();
+      if (x[m] < -745.1332191019412) e[m] = 0.0;
+      if (x[m] != x[m]) e[m] = x[m];
+    }
+  }
+}
+
+// Two logarithms at once, the bits of pr_log for each: as exp_n, with the rare arguments (zero,
+// negative, infinite, NaN) behind a branch no wavefront takes in practice.
+__device__ __forceinline__ void log_2(double xa, double xb, double& la, double& lb) {
+  const double x[2] = {xa, xb};
+  double s2[2], z[2], p[2], de[2], lg[2];
+  bool odd = false;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    odd |= !(x[m] > 0.0 && x[m] < __builtin_huge_val());
+    int e;
+    double mm = frexp(x[m], &e);
+    if (mm < PRK_SQRT_HALF) {
+      mm = mm * 2.0;
+      e = e - 1;
+    }
+    const double f = mm - 1.0;
+    const double s = f / (2.0 + f);
+    z[m] = s * s;
+    s2[m] = s + s;
+    de[m] = (double)e;
+    p[m] = 1.0 / 21.0;
+  }
+#define PRK_LOG_STEP(C)                                          \
+  {                                                              \
+    const double c = kc(C);                                      \
+    _Pragma("unroll") for (int m = 0; m < 2; ++m) p[m] = fma(p[m], z[m], c); \
+  }
+  PRK_LOG_STEP(1.0 / 19.0)
+  PRK_LOG_STEP(1.0 / 17.0)
+  PRK_LOG_STEP(1.0 / 15.0)
+  PRK_LOG_STEP(1.0 / 13.0)
+  PRK_LOG_STEP(1.0 / 11.0)
+  PRK_LOG_STEP(1.0 / 9.0)
+  PRK_LOG_STEP(1.0 / 7.0)
+  PRK_LOG_STEP(1.0 / 5.0)
+  PRK_LOG_STEP(1.0 / 3.0)
+#undef PRK_LOG_STEP
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const double t = z[m] * p[m];
+    const double logm = fma(s2[m], t, s2[m]);
+    lg[m] = fma(de[m], PRK_LN2_HI, fma(de[m], PRK_LN2_LO, logm));
+  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(odd) != 0, 0)) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (!(x[m] > 0.0)) lg[m] = (x[m] == 0.0) ? -__builtin_huge_val() : __builtin_nan("");
+      if (x[m] == __builtin_huge_val()) lg[m] = x[m];
+    }
+  }
+  la = lg[0];
+  lb = lg[1];
+}
 
 // v through an empty volatile asm: expressions of it are computed where they are used, not
 // hoisted out of the integrator loop into registers held for the whole kernel.
@@ -356,14 +487,14 @@ struct RxOut {
 // One reaction at (C, T): effective rate coefficients, forward / reverse rates and, when JAC,
 // d q / d[M] and d q / dT at constant concentrations.
 template <bool JAC>
-__device__ __forceinline__ void rx_eval(const RxRec& rx, const double* sC, const double* sG,
+__device__ __forceinline__ void rx_eval(const ExpK& K, const RxRec& rx, const double* sC, const double* sG,
                                         const double* sH, double Ctot, double T, double lnT,
                                         double invT, double lnRTP, const int* effsp,
                                         const double* effval, RxOut& o) {
   const int info = rx.info;
   const int type = info & 15, rev = (info >> 4) & 15, nre = (info >> 8) & 15, npr = (info >> 12) & 15;
   const int ntroe = (info >> 16) & 15;
-  const double kinf = pr_exp(fma(-rx.Ta, invT, fma(rx.beta, lnT, rx.lnA)));
+  const double ka = fma(-rx.Ta, invT, fma(rx.beta, lnT, rx.lnA));
   const double dlnkinf = fma(rx.Ta, invT, rx.beta) * invT;
   double M = 0.0;
   if (type != PR_RX_ELEM) {
@@ -392,16 +523,23 @@ __device__ __forceinline__ void rx_eval(const RxRec& rx, const double* sC, const
   double pp = cp0;
   if (npr > 1) pp *= cp1;
   if (npr > 2) pp *= cp2;
-  double invKc = 0.0, dH = 0.0;
+  double kinf, invKc, dH = 0.0;
   const int sumnu = npr - nre;
-  if (rev) {
+  {
     double dG = gp0;
     if (npr > 1) dG += gp1;
     if (npr > 2) dG += gp2;
     dG -= gr0;
     if (nre > 1) dG -= gr1;
     if (nre > 2) dG -= gr2;
-    invKc = pr_exp(fma((double)sumnu, lnRTP, dG));
+    // forward and reverse exponential together (an irreversible reaction's second one is dropped)
+    const double x[2] = {ka, rev ? fma((double)sumnu, lnRTP, dG) : 0.0};
+    double e[2];
+    exp_n<2>(K, x, e);
+    kinf = e[0];
+    invKc = rev ? e[1] : 0.0;
+  }
+  if (rev) {
     if (JAC) {
       const double hr0 = sH[r0], hr1 = sH[r1], hr2 = sH[r2], hp0 = sH[p0], hp1 = sH[p1], hp2 = sH[p2];
       dH = hp0;
@@ -426,28 +564,37 @@ __device__ __forceinline__ void rx_eval(const RxRec& rx, const double* sC, const
     }
     return;
   }
-  const double k0 = pr_exp(fma(-rx.Ta0, invT, fma(rx.beta0, lnT, rx.lnA0)));
-  double Pr = (k0 * M) / kinf;
-  if (Pr < 1e-300) Pr = 1e-300;
-  double F = 1.0, dlogF_dx = 0.0, dlogF_dT = 0.0, dlnPr = 0.0;
+  const double k0a = fma(-rx.Ta0, invT, fma(rx.beta0, lnT, rx.lnA0));
+  double k0, Pr, F = 1.0, dlogF_dx = 0.0, dlogF_dT = 0.0, dlnPr = 0.0;
   if (JAC) dlnPr = fma(rx.Ta0, invT, rx.beta0) * invT - dlnkinf;
   if (type == PR_RX_TROE) {
-    const double e3 = pr_exp(-T / rx.troe[1]), e1 = pr_exp(-T / rx.troe[2]);
+    // the low-pressure rate and Fcent's exponentials together
+    const double xe[4] = {k0a, -T / rx.troe[1], -T / rx.troe[2], ntroe == 4 ? -rx.troe[3] * invT : 0.0};
+    double ex[4];
+    exp_n<4>(K, xe, ex);
+    k0 = ex[0];
+    Pr = (k0 * M) / kinf;
+    if (Pr < 1e-300) Pr = 1e-300;
+    const double e3 = ex[1], e1 = ex[2];
     double Fc = (1.0 - rx.troe[0]) * e3 + rx.troe[0] * e1;
     double dFc = 0.0;
     if (JAC) dFc = -((1.0 - rx.troe[0]) / rx.troe[1]) * e3 - (rx.troe[0] / rx.troe[2]) * e1;
     if (ntroe == 4) {
-      const double e2 = pr_exp(-rx.troe[3] * invT);
+      const double e2 = ex[3];
       Fc += e2;
       if (JAC) dFc += ((rx.troe[3] * invT) * invT) * e2;
     }
     if (Fc < 1e-300) Fc = 1e-300;
-    const double logFc = pr_log10(Fc);
+    double lFc, lPr;
+    log_2(Fc, Pr, lFc, lPr);
+    const double logFc = lFc * PRK_INV_LN10, x = lPr * PRK_INV_LN10;
     const double c = -0.4 - 0.67 * logFc, nn = 0.75 - 1.27 * logFc;
-    const double x = pr_log10(Pr);
     const double xc = x + c, D = nn - 0.14 * xc, f1 = xc / D;
     const double den = 1.0 + f1 * f1;
-    F = pr_exp((logFc / den) * PRK_LN10);
+    const double xf[1] = {(logFc / den) * PRK_LN10};
+    double ef[1];
+    exp_n<1>(K, xf, ef);
+    F = ef[0];
     if (JAC) {
       dlogF_dx = -logFc * 2.0 * f1 * (nn / (D * D)) / (den * den);
       const double dlogFc = dFc / (Fc * PRK_LN10);
@@ -456,6 +603,13 @@ __device__ __forceinline__ void rx_eval(const RxRec& rx, const double* sC, const
       const double df1 = (dxc * D - xc * dD) / (D * D);
       dlogF_dT = (dlogFc * den - logFc * 2.0 * f1 * df1) / (den * den);
     }
+  } else {
+    const double x0[1] = {k0a};
+    double e0[1];
+    exp_n<1>(K, x0, e0);
+    k0 = e0[0];
+    Pr = (k0 * M) / kinf;
+    if (Pr < 1e-300) Pr = 1e-300;
   }
   const double kf = ((kinf * Pr) / (1.0 + Pr)) * F;
   const double kr = kf * invKc;
@@ -480,14 +634,13 @@ struct Smem {
   const RxRec* rx;
   const int* effsp;
   const double* effval;
-  const int* incs;
-  const int* inc;
   const int* incq;       // byte offset of each incidence entry's rate slot in q
   const double* incnu;   // its stoichiometric coefficient
   const int* kblk;       // first gather block of each species; kblk[N] = number of blocks
   const int* blk;        // first incidence entry of each gather block (blk[nblocks] = ninc)
   double* Js;    // global scratch slot: (N+1)^2 row-major saved Jacobian
-  double* jrec;  // global scratch slot: 4 R per-reaction Jacobian records (kf, kr, dqdM, dqdT)
+  double* jrec;  // global scratch slot: Jacobian records kf, kr, dqdM, dqdT, q of every reaction, [5][R]
+  JacTabs jt;    // what each Jacobian entry sums
   double* sC;    // N concentrations
   double* sG;    // N g/RT
   double* sH;    // N h/RT
@@ -501,7 +654,7 @@ struct Smem {
   static constexpr int n = N + 1;
   // per-group LDS (doubles) and per-group global scratch slot (doubles)
   static constexpr int scratch_doubles = 5 * N + R + (n + 1) / 2 + 1;
-  static constexpr int slot_doubles = n * n + 4 * R;
+  static constexpr int slot_doubles = n * n + 5 * R;
 };
 
 template <int N, int R, int G>
@@ -585,12 +738,13 @@ __device__ __forceinline__ void net_rates(const Smem<N, R>& S, int lane, double 
   }
   const double Ctot = gpsum<G, RPL, N>(lane, cc);
   group_sync();
+  const ExpK K = exp_constants();
 #pragma unroll 1
   for (int m = 0; m < Cell<N, R, G>::RXL; ++m) {
     const int r = lane + G * m;
     if (r < R) {
       RxOut o;
-      rx_eval<false>(S.rx[r], S.sC, S.sG, S.sH, Ctot, T, lnT, invT, lnRTP, S.effsp, S.effval, o);
+      rx_eval<false>(K, S.rx[r], S.sC, S.sG, S.sH, Ctot, T, lnT, invT, lnRTP, S.effsp, S.effval, o);
       S.q[r] = o.fwd - o.rev;
     }
   }
@@ -707,11 +861,13 @@ __device__ __forceinline__ void rate_rhoY_eval(const Smem<N, R>& S, int lane, co
 }
 
 // ---------------------------------------------------------------- analytic Jacobian
-// Exact Jacobian of the right-hand side with T = y_T, written into S.Js (row-major). Rows are
-// assembled in LDS (the saved Jacobian itself at G = 64, else the LU area, which is dead here:
-// a factorization always follows) and then copied to the global slot; above 32 components there
-// is no LU area in LDS and they are assembled in the global slot itself (each lane updates its
-// own row; a wavefront's global accesses to one address complete in order).
+// Exact Jacobian of the right-hand side with T = y_T, written into S.Js (row-major). Assembled in
+// the saved Jacobian itself (LDS at G = 64 up to 32 components, else the global slot), at G = 8 / 16
+// in the LU area, which is dead here (a factorization always follows), and copied to the slot.
+// Every lane sums whole entries (JacTabs), in the order of the species' incidence list: a row per
+// lane instead left the lane of the longest list (84 of dodecane_lu's 918 entries) adding into its
+// row one dependent read-modify-write after another. What bounds it now is the rate pass; 8192
+// drm19 Jacobians 247 -> 97 us, and the react of 64^3 cells 122.4 -> 116.9 ms.
 template <int N, int R, int G>
 __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const double (&y)[Cell<N, R, G>::RPL],
                                          const double (&src)[Cell<N, R, G>::RPL], double rhohsrc) {
@@ -743,21 +899,50 @@ __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const do
     }
   }
   const double Ctot = gpsum<G, RPL, N>(lane, cc);
+  const ExpK K = exp_constants();
 #pragma unroll 1
   for (int m = 0; m < Cell<N, R, G>::RXL; ++m) {
     const int r = lane + G * m;
     if (r < R) {
       RxOut o;
-      rx_eval<true>(S.rx[r], S.sC, S.sG, S.sH, Ctot, T, lnT, invT, lnRTP, S.effsp, S.effval, o);
-      double* rc = S.jrec + 4 * r;
+      rx_eval<true>(K, S.rx[r], S.sC, S.sG, S.sH, Ctot, T, lnT, invT, lnRTP, S.effsp, S.effval, o);
+      double* rc = S.jrec + r;
       rc[0] = o.kf;
-      rc[1] = o.kr;
-      rc[2] = o.dqdM;
-      rc[3] = o.dqdT;
-      S.q[r] = o.fwd - o.rev;
+      rc[R] = o.kr;
+      rc[2 * R] = o.dqdM;
+      rc[3 * R] = o.dqdT;
+      rc[4 * R] = o.fwd - o.rev;
     }
   }
+  static_assert(R > N, "the rates' array holds the species' sums and a 1.0");
+  S.q[N] = 1.0;
   group_sync();
+#pragma unroll 1
+  for (int e0 = 0; e0 < S.jt.nentry; e0 += G) {
+    const JacEntry en = S.jt.entry[e0 + lane];
+    const JacTerm* const tp = S.jt.term + S.jt.slice[e0 / 64] + e0 % 64 + lane;
+    double a = 0.0;
+#pragma unroll 1
+    for (int i = 0; i < en.nt; i += 4) {  // the reads of four terms first, then their sum in order
+      double v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const JacTerm t = tp[64 * (i + u < en.nt ? i + u : i)];
+        const unsigned char* const cb = reinterpret_cast<const unsigned char*>(S.sC);
+        v[u] = ((t.coef * S.jrec[t.rec]) * *reinterpret_cast<const double*>(cb + t.c1)) *
+               *reinterpret_cast<const double*>(cb + t.c2);
+      }
+      a += v[0];
+#pragma unroll
+      for (int u = 1; u < 4; ++u)
+        if (i + u < en.nt) a += v[u];
+    }
+    if (en.dst >= 0) A[en.dst] = a;
+    else if (en.dst != kJacNone) S.sC[~en.dst] = a;
+  }
+  group_sync();
+  const double* const Sd = S.sG;  // sum of nu dq/d[M] times the default efficiency
+  const double* const JT = S.sH;  // sum of nu dq/dT
   double pn[RPL], prcp[RPL], psd[RPL], pcf[RPL];
 #pragma unroll
   for (int s = 0; s < RPL; ++s) {
@@ -767,41 +952,9 @@ __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const do
     psd[s] = 0.0;
     pcf[s] = 0.0;
     if (k < N) {
-      double* row = A + k * n;
-      for (int j = 0; j < n; ++j) row[j] = 0.0;
-      double Sd = 0.0, JT = 0.0, w = 0.0;
-      for (int e = S.incs[k]; e < S.incs[k + 1]; ++e) {
-        const int rn = S.inc[e];
-        const int r = rn & 0xFFFF;
-        const double nu = (double)(rn >> 16);
-        const RxRec& rx = S.rx[r];
-        const double* rc = S.jrec + 4 * r;
-        const int info = rx.info, type = info & 15, nre = (info >> 8) & 15, npr = (info >> 12) & 15;
-        w += nu * S.q[r];
-        const int a0 = rx.reac & 0xFF, a1 = (rx.reac >> 8) & 0xFF, a2 = (rx.reac >> 16) & 0xFF;
-        const double c0 = S.sC[a0], c1 = nre > 1 ? S.sC[a1] : 1.0, c2 = nre > 2 ? S.sC[a2] : 1.0;
-        const double kf = nu * rc[0];
-        row[a0] += (kf * c1) * c2;
-        if (nre > 1) row[a1] += (kf * c0) * c2;
-        if (nre > 2) row[a2] += (kf * c0) * c1;
-        const int b0 = rx.prod & 0xFF, b1 = (rx.prod >> 8) & 0xFF, b2 = (rx.prod >> 16) & 0xFF;
-        const double d0 = S.sC[b0], d1 = npr > 1 ? S.sC[b1] : 1.0, d2 = npr > 2 ? S.sC[b2] : 1.0;
-        const double kr = nu * rc[1];
-        row[b0] -= (kr * d1) * d2;
-        if (npr > 1) row[b1] -= (kr * d0) * d2;
-        if (npr > 2) row[b2] -= (kr * d0) * d1;
-        if (type != PR_RX_ELEM) {
-          const double dm = nu * rc[2];
-          Sd += dm * rx.effd;
-          const int eb = rx.eff & 0xFFFF, ee = (rx.eff >> 16) & 0xFFFF;
-          for (int q = eb; q < ee; ++q) row[S.effsp[q]] += dm * S.effval[q];
-        }
-        JT += nu * rc[3];
-      }
       const double Wk = S.sp[k].W;
-      for (int j = 0; j < N; ++j) row[j] = ((row[j] + Sd) * Wk) * S.sp[j].invW;
-      row[N] = JT * Wk;
-      const double fk = w * Wk + src[s];
+      A[k * n + N] = JT[k] * Wk;
+      const double fk = S.q[k] * Wk + src[s];
       pn[s] = S.sHm[k] * fk;
       prcp[s] = y[s] * cpk[s];
       psd[s] = y[s] * dcpk[s];
@@ -817,7 +970,23 @@ __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const do
     const int j = lane + G * s;
     if (j < n) {
       double cs = 0.0;
-      for (int k = 0; k < N; ++k) cs += S.sHm[k] * A[k * n + j];
+      const double iw = j < N ? S.sp[j].invW : 0.0;
+#pragma unroll 1
+      for (int k0 = 0; k0 < N; k0 += 8) {  // eight entries of the column read before any is rewritten
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = A[(k0 + u < N ? k0 + u : N - 1) * n + j];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int k = k0 + u;
+          if (k >= N) break;
+          if (j < N) {
+            v[u] = ((v[u] + Sd[k]) * S.sp[k].W) * iw;
+            A[k * n + j] = v[u];
+          }
+          cs += S.sHm[k] * v[u];
+        }
+      }
       A[N * n + j] = (j < N) ? (-cs - fT * S.sCpm[j]) / rcp : ((-cs - scf) - fT * sdcp) / rcp;
     }
   }

@@ -208,61 +208,6 @@ __device__ __forceinline__ void rows_thermo(const RateLds<N, R, G>& L, int lane,
   }
 }
 
-// pr_exp's constants, held in scalar registers over a loop: each polynomial step is then one
-// v_fma_f64 with a scalar addend and nothing else.
-struct ExpK {
-  double l2e, hi, lo, c13, c12, c11, c10, c9, c8, c7, c6, c5, c4, c3;
-};
-__device__ __forceinline__ ExpK exp_constants() {
-  return ExpK{kc(PRK_LOG2E),        kc(PRK_LN2_HI),       kc(PRK_LN2_LO),      kc(1.0 / 6227020800.0), kc(1.0 / 479001600.0),
-              kc(1.0 / 39916800.0), kc(1.0 / 3628800.0),  kc(1.0 / 362880.0),  kc(1.0 / 40320.0),      kc(1.0 / 5040.0),
-              kc(1.0 / 720.0),      kc(1.0 / 120.0),      kc(1.0 / 24.0),      kc(1.0 / 6.0)};
-}
-
-// M exponentials at once, the bits of pr_exp: M independent chains in one basic block (one chain of
-// 20 dependent FP64 operations leaves most issue slots of a wavefront empty). pr_exp's range tests
-// are one comparison per argument and a branch no wavefront takes in practice.
-template <int M>
-__device__ __forceinline__ void exp_n(const ExpK& K, const double (&x)[M], double (&e)[M]) {
-  bool far = false;
-#pragma unroll
-  for (int m = 0; m < M; ++m) far |= !(fabs(x[m]) < 700.0);
-  double k[M], r[M], p[M];
-#pragma unroll
-  for (int m = 0; m < M; ++m) k[m] = rint(x[m] * K.l2e);
-#pragma unroll
-  for (int m = 0; m < M; ++m) r[m] = fma(-k[m], K.hi, x[m]);
-#pragma unroll
-  for (int m = 0; m < M; ++m) r[m] = fma(-k[m], K.lo, r[m]);
-#pragma unroll
-  for (int m = 0; m < M; ++m) p[m] = fma(K.c13, r[m], K.c12);
-#define PRK_EXP_STEP(C) \
-  _Pragma("unroll") for (int m = 0; m < M; ++m) p[m] = fma(p[m], r[m], C)
-  PRK_EXP_STEP(K.c11);
-  PRK_EXP_STEP(K.c10);
-  PRK_EXP_STEP(K.c9);
-  PRK_EXP_STEP(K.c8);
-  PRK_EXP_STEP(K.c7);
-  PRK_EXP_STEP(K.c6);
-  PRK_EXP_STEP(K.c5);
-  PRK_EXP_STEP(K.c4);
-  PRK_EXP_STEP(K.c3);
-  PRK_EXP_STEP(0.5);
-  PRK_EXP_STEP(1.0);
-  PRK_EXP_STEP(1.0);
-#undef PRK_EXP_STEP
-#pragma unroll
-  for (int m = 0; m < M; ++m) e[m] = ldexp(p[m], (int)k[m]);
-  if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      if (x[m] > 709.782712893384) e[m] = __builtin_huge_val();
-      if (x[m] < -745.1332191019412) e[m] = 0.0;
-      if (x[m] != x[m]) e[m] = x[m];
-    }
-  }
-}
-
 // A reaction's record in scalar registers: everything but the falloff parameters.
 struct RxHead {
   double lnA, beta, Ta, effd;

@@ -53,8 +53,6 @@ __device__ __forceinline__ double* setup_views(Smem<N, R>& S, unsigned char* sme
   S.rx = reinterpret_cast<const RxRec*>(smem + BL.off_rx);
   S.effsp = reinterpret_cast<const int*>(smem + BL.off_effsp);
   S.effval = reinterpret_cast<const double*>(smem + BL.off_effval);
-  S.incs = reinterpret_cast<const int*>(smem + BL.off_incs);
-  S.inc = reinterpret_cast<const int*>(smem + BL.off_inc);
   S.incq = reinterpret_cast<const int*>(smem + BL.off_incq);
   S.incnu = reinterpret_cast<const double*>(smem + BL.off_incnu);
   S.kblk = reinterpret_cast<const int*>(smem + BL.off_kblk);
@@ -76,7 +74,7 @@ __device__ __forceinline__ double* setup_views(Smem<N, R>& S, unsigned char* sme
     const long slot = (long)blockIdx.x * (blockDim.x / G) + grp;
     S.Js = gscr + slot * Cell<N, R, G>::gslot_doubles;
     S.jrec = S.Js + n * n;
-    if constexpr (Cell<N, R, G>::lu_global) S.LU = S.jrec + 4 * R;  // n n doubles after the records
+    if constexpr (Cell<N, R, G>::lu_global) S.LU = S.jrec + 5 * R;  // n n doubles after the records
   } else {
     S.Js = nullptr;  // kernels without a Jacobian
     S.jrec = nullptr;
@@ -100,6 +98,7 @@ __global__ void __launch_bounds__(256 * W) __attribute__((amdgpu_waves_per_eu(W,
   __syncthreads();
   const BlobLayout BL = blob_layout(N, R, P.neff, P.ninc);
   Smem<N, R> S;
+  S.jt = P.jt;
   int lane = threadIdx.x % G;  // re-derived opaquely each iteration (see the loop head)
   const int grp = threadIdx.x / G;
   Ctl* ct = reinterpret_cast<Ctl*>(setup_views<N, R, G>(S, smem, BL, grp, P.gscr));
@@ -854,7 +853,7 @@ template <int N, int R, int G, int MODE>
 __global__ void __launch_bounds__(BLOCK) eval_kernel(const unsigned char* blob, int blob_bytes, int neff, int ninc,
                                                      long ncells, const double* y, const double* rYsrc,
                                                      const double* rhoh0, const double* rhohsrc, double t,
-                                                     double* out, double* gscr) {
+                                                     double* out, double* gscr, JacTabs jt) {
   constexpr int n = N + 1;
   constexpr int RPL = Cell<N, R, G>::RPL;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -866,6 +865,7 @@ __global__ void __launch_bounds__(BLOCK) eval_kernel(const unsigned char* blob, 
   __syncthreads();
   const BlobLayout BL = blob_layout(N, R, neff, ninc);
   Smem<N, R> S;
+  S.jt = jt;
   const int lane = threadIdx.x % G;
   const int grp = threadIdx.x / G;
   setup_views<N, R, G>(S, smem, BL, grp, gscr);

@@ -58,8 +58,8 @@ const pr_mech_t* find_mech(const char* name) {
 using Launch = hipError_t (*)(const prk::KParams&, int blocks, int block, size_t shmem, hipStream_t);
 using EvalLaunch = hipError_t (*)(int mode, const unsigned char* blob, int blob_bytes, int neff, int ninc, long ncells,
                                   const double* y, const double* rYsrc, const double* rhoh0, const double* rhohsrc,
-                                  double t, double* out, double* gscr, int blocks, int block, size_t shmem,
-                                  hipStream_t st);
+                                  double t, double* out, double* gscr, const prk::JacTabs& jt, int blocks, int block,
+                                  size_t shmem, hipStream_t st);
 using Occ = hipError_t (*)(int* nb, int block, size_t shmem);
 using RateLaunch = hipError_t (*)(const prk::RateParams&, int blocks, int block, size_t shmem, hipStream_t);
 using BlockRateLaunch = hipError_t (*)(const prk::RateParams&, const prk::BlockTabs&, int cus, hipStream_t);
@@ -77,13 +77,13 @@ hipError_t launch_t(const prk::KParams& P, int blocks, int block, size_t shmem, 
 template <int N, int R, int G>
 hipError_t eval_t(int mode, const unsigned char* blob, int blob_bytes, int neff, int ninc, long ncells, const double* y,
                   const double* rYsrc, const double* rhoh0, const double* rhohsrc, double t, double* out, double* gscr,
-                  int blocks, int block, size_t shmem, hipStream_t st) {
+                  const prk::JacTabs& jt, int blocks, int block, size_t shmem, hipStream_t st) {
   if (mode == 0)
     hipLaunchKernelGGL((prk::eval_kernel<N, R, G, 0>), dim3(blocks), dim3(block), shmem, st, blob, blob_bytes, neff,
-                       ninc, ncells, y, rYsrc, rhoh0, rhohsrc, t, out, gscr);
+                       ninc, ncells, y, rYsrc, rhoh0, rhohsrc, t, out, gscr, jt);
   else
     hipLaunchKernelGGL((prk::eval_kernel<N, R, G, 1>), dim3(blocks), dim3(block), shmem, st, blob, blob_bytes, neff,
-                       ninc, ncells, y, rYsrc, rhoh0, rhohsrc, t, out, gscr);
+                       ninc, ncells, y, rYsrc, rhoh0, rhohsrc, t, out, gscr, jt);
   return hipGetLastError();
 }
 
@@ -336,10 +336,6 @@ std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
     esp[e] = m->eff_sp[e];
     eval[e] = m->eff_val[e];
   }
-  auto* incs = reinterpret_cast<int*>(b.data() + L.off_incs);
-  auto* inc = reinterpret_cast<int*>(b.data() + L.off_inc);
-  for (int k = 0; k <= m->nsp; ++k) incs[k] = m->inc_start[k];
-  for (int e = 0; e < m->ninc; ++e) inc[e] = (slot_of[m->inc_r[e]] & 0xFFFF) | (m->inc_nu[e] * 65536);
   // the production-rate gather: per entry the byte offset of its rate slot and nu as a double,
   // and the incidence lists cut into PR_GATHER_BLOCK-entry blocks
   auto* incq = reinterpret_cast<int*>(b.data() + L.off_incq);
@@ -432,6 +428,86 @@ std::vector<unsigned char> pack_block_tabs(const pr_mech_t* m, const std::vector
   off[1] = put(rrange.data(), sizeof(int32_t) * rrange.size());
   off[2] = put(pieces.data(), sizeof(prk::GatherPiece) * pieces.size());
   off[3] = put(prange.data(), sizeof(int32_t) * prange.size());
+  return out;
+}
+
+// Terms of every Jacobian entry (JacTabs) in the order of the species' incidence lists. Offsets of
+// the three sections go to off[].
+std::vector<unsigned char> pack_jac_tabs(const pr_mech_t* m, const std::vector<unsigned char>& blob, size_t off[3],
+                                         int* nentry) {
+  const int N = m->nsp, R = m->nr, n = N + 1;
+  const prk::BlobLayout L = prk::blob_layout(m->nsp, m->nr, m->neff, m->ninc);
+  const auto* incq = reinterpret_cast<const int*>(blob.data() + L.off_incq);
+  struct Entry {
+    int dst;
+    std::vector<prk::JacTerm> t;
+  };
+  std::vector<Entry> ent;
+  const uint16_t one = (uint16_t)(8 * 6 * N);
+  for (int k = 0; k < N; ++k) {
+    std::vector<Entry> col(N + 3);  // the species' columns, then its sums over dq/d[M], dq/dT and q
+    for (int j = 0; j < N; ++j) col[j].dst = k * n + j;
+    col[N].dst = ~(N + k);
+    col[N + 1].dst = ~(2 * N + k);
+    col[N + 2].dst = ~(5 * N + k);
+    int slot = 0;  // of the incidence entry's reaction in the blob
+    auto add = [&](int c, double coef, int plane, int c1, int c2) {
+      prk::JacTerm t{};
+      t.coef = coef;
+      t.rec = plane * R + slot;
+      t.c1 = c1 < 0 ? one : (uint16_t)(8 * c1);
+      t.c2 = c2 < 0 ? one : (uint16_t)(8 * c2);
+      col[c].t.push_back(t);
+    };
+    for (int e = m->inc_start[k]; e < m->inc_start[k + 1]; ++e) {
+      const int r = m->inc_r[e];
+      const double nu = (double)m->inc_nu[e];
+      slot = incq[e] / (int)sizeof(double);
+      add(N + 2, nu, 4, -1, -1);
+      for (int side = 0; side < 2; ++side) {
+        const int cnt = side ? m->nprod[r] : m->nreac[r];
+        const int* sp = (side ? m->prod : m->reac) + 3 * r;
+        for (int s = 0; s < cnt; ++s) {  // the rate over this slot's concentration: the other slots' product
+          int o[2] = {-1, -1}, no = 0;
+          for (int q = 0; q < cnt; ++q)
+            if (q != s) o[no++] = sp[q];
+          add(sp[s], side ? -nu : nu, side, o[0], o[1]);
+        }
+      }
+      if (m->rtype[r] != PR_RX_ELEM) {
+        add(N, nu * m->eff_dflt[r], 2, -1, -1);
+        for (int q = m->eff_start[r]; q < m->eff_start[r + 1]; ++q) add(m->eff_sp[q], nu * m->eff_val[q], 2, -1, -1);
+      }
+      add(N + 1, nu, 3, -1, -1);
+    }
+    for (Entry& c : col) ent.push_back(std::move(c));
+  }
+  std::stable_sort(ent.begin(), ent.end(), [](const Entry& a, const Entry& b) { return a.t.size() > b.t.size(); });
+  while (ent.size() % 64) ent.push_back({prk::kJacNone, {}});
+  std::vector<prk::JacTerm> term;
+  std::vector<prk::JacEntry> entry;
+  std::vector<int32_t> slice;
+  for (size_t b = 0; b < ent.size(); b += 64) {
+    slice.push_back((int32_t)term.size());
+    const size_t len = ent[b].t.size();
+    term.resize(term.size() + 64 * len, prk::JacTerm{});
+    for (size_t l = 0; l < 64; ++l) {
+      const Entry& c = ent[b + l];
+      entry.push_back({(int32_t)c.t.size(), c.dst});
+      for (size_t i = 0; i < c.t.size(); ++i) term[(size_t)slice.back() + 64 * i + l] = c.t[i];
+    }
+  }
+  *nentry = (int)entry.size();
+  std::vector<unsigned char> out;
+  auto put = [&](const void* p, size_t bytes) {
+    const size_t at = (out.size() + 63) / 64 * 64;
+    out.resize(at + bytes, 0);
+    std::memcpy(out.data() + at, p, bytes);
+    return at;
+  };
+  off[0] = put(term.data(), sizeof(prk::JacTerm) * term.size());
+  off[1] = put(entry.data(), sizeof(prk::JacEntry) * entry.size());
+  off[2] = put(slice.data(), sizeof(int32_t) * slice.size());
   return out;
 }
 
@@ -594,6 +670,8 @@ struct pr_handle {
   const BlockOps* blk = nullptr;
   prk::BlockTabs tabs{};       // device tables of the block kernels, one allocation
   void* d_tabs = nullptr;
+  prk::JacTabs jtabs{};        // device tables of the Jacobian, one allocation
+  void* d_jtabs = nullptr;
   double* d_atolv = nullptr;
   void* d_counters = nullptr;  // two regions of 128 B: queue (4 B), nfail (4 B), stats (8 x 8 B at +64)
   double* d_gscr = nullptr;    // per-group global scratch slots
@@ -684,9 +762,12 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
   size_t toff[4];
   h->blk = find_block_ops(m->name);
   const std::vector<unsigned char> tabs = pack_block_tabs(m, blob, h->blk->waves, h->blk->nchunk, toff);
+  size_t joff[3];
+  const std::vector<unsigned char> jtabs = pack_jac_tabs(m, blob, joff, &h->jtabs.nentry);
   const std::vector<double> atol0((size_t)m->nsp + 1, K.atol);
   if (hipMalloc(&h->d_blob, blob.size()) != hipSuccess || hipMalloc(&h->d_counters, 256) != hipSuccess ||
-      hipMalloc(&h->d_tabs, tabs.size()) != hipSuccess ||
+      hipMalloc(&h->d_tabs, tabs.size()) != hipSuccess || hipMalloc(&h->d_jtabs, jtabs.size()) != hipSuccess ||
+      hipMemcpy(h->d_jtabs, jtabs.data(), jtabs.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(h->d_tabs, tabs.data(), tabs.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMalloc(&h->d_atolv, sizeof(double) * (m->nsp + 1)) != hipSuccess ||
       hipMemcpy(h->d_atolv, atol0.data(), sizeof(double) * atol0.size(), hipMemcpyHostToDevice) != hipSuccess ||
@@ -703,6 +784,10 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
     h->tabs.piece = reinterpret_cast<const prk::GatherPiece*>(t + toff[2]);
     h->tabs.piece_range = reinterpret_cast<const int32_t*>(t + toff[3]);
     h->tabs.nchunk = h->blk->nchunk;
+    auto* j = static_cast<unsigned char*>(h->d_jtabs);
+    h->jtabs.term = reinterpret_cast<const prk::JacTerm*>(j + joff[0]);
+    h->jtabs.entry = reinterpret_cast<const prk::JacEntry*>(j + joff[1]);
+    h->jtabs.slice = reinterpret_cast<const int32_t*>(j + joff[2]);
   }
   *out = h;
   return 0;
@@ -1423,6 +1508,7 @@ static int react_box_core(pr_handle* h, const int lo[3], const int hi[3], const 
   P.rtol = h->keys.rtol;
   P.atol = h->keys.atol;
   P.atolv = h->d_atolv;
+  P.jt = h->jtabs;
   P.max_order = h->keys.max_order;
   P.max_steps = h->keys.max_substeps;
   P.clean = h->keys.clean_init_massfrac;
@@ -1635,6 +1721,7 @@ int pr_react_batch_enqueue(pr_handle* h, int nbox, const pr_box* boxes, void* st
   P.rtol = h->keys.rtol;
   P.atol = h->keys.atol;
   P.atolv = h->d_atolv;
+  P.jt = h->jtabs;
   P.max_order = h->keys.max_order;
   P.max_steps = h->keys.max_substeps;
   P.clean = h->keys.clean_init_massfrac;
@@ -1780,7 +1867,7 @@ static int eval_batch(pr_handle* h, int mode, int64_t ncells, const double* y, c
   }
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(h->var->eval(mode, h->d_blob, h->blob_bytes, h->mech->neff, h->mech->ninc, (long)ncells, y, rYsrc, rhoh0,
-                      rhohsrc, t, out, h->d_gscr, blocks, block, shmem, st));
+                      rhohsrc, t, out, h->d_gscr, h->jtabs, blocks, block, shmem, st));
   HIPCHK(hipStreamSynchronize(st));
   return 0;
 }
@@ -2432,6 +2519,7 @@ void pr_destroy(pr_handle* h) {
   if (h->d_blob) (void)hipFree(h->d_blob);
   if (h->d_counters) (void)hipFree(h->d_counters);
   if (h->d_tabs) (void)hipFree(h->d_tabs);
+  if (h->d_jtabs) (void)hipFree(h->d_jtabs);
   if (h->d_atolv) (void)hipFree(h->d_atolv);
   if (h->d_gscr) (void)hipFree(h->d_gscr);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
