@@ -1,6 +1,6 @@
-// Equation-of-state box kernels around the chemistry advance, MKS Array4 views, one thread per
-// cell (cells fastest, so every species row of the box is read and written coalesced; the
-// species records are staged in LDS and read by all lanes at once):
+// Equation-of-state box kernels around the chemistry advance, MKS Array4 views (cells fastest, so
+// every species row of the box is read and written coalesced; the species records are staged in
+// LDS), one thread per cell except setTemperature (a quad or eight lanes per cell):
 //  * setTemperature  (Source/PeleLMeX_Eos.cpp:218-240 -> getTfromHY, Source/PeleLMeX_K.H:700-723):
 //    rhoinv = 1 / rho, Y = rhoY * rhoinv, h = rhoH * rhoinv * 1e4, T = HY2T(h, Y) from the stored
 //    T - the reactor's own iteration and sums (hy2t), so the temperature is the one its
@@ -16,7 +16,7 @@
 
 #include <cfloat>
 
-#include "react_kernel.h"
+#include "block_rates.h"
 
 namespace prk {
 
@@ -29,54 +29,6 @@ struct EosParams {
   const unsigned char* blob;
   int blob_bytes, neff, ninc;
 };
-
-// hy2t of the reactor (bdf_kernel.h) by one thread: the same Newton iteration, with the mixture
-// enthalpy and heat capacity summed over the canonical pairwise tree of the reactor's component
-// sums (64 zero-padded slots: pairs, pairs of pairs, ...). The tree is evaluated as the slots are
-// formed, keeping one pending left subtree per level, so only six partial sums per quantity are
-// live; Y_k = rhoY_k / rho is re-read from the cell's row at each iteration.
-template <int N>
-__device__ __forceinline__ double hy2t_cell(const SpRec* sp, const double* rY, long ns, double rhoinv, double h,
-                                            double T) {
-  static_assert(N <= 64, "at most 64 components");
-  for (int it = 0; it < 20; ++it) {
-    const double invT = 1.0 / T;
-    double sh[6], sc[6], hm = 0.0, cpm = 0.0;
-#pragma unroll 1
-    for (int s = 0; s < 64; ++s) {
-      double a = 0.0, b = 0.0;
-      if (s < N) {
-        const double Y = rY[(long)s * ns] * rhoinv;
-        double cpR, hRT;
-        nasa_hcp(sp[s], T, invT, cpR, hRT);
-        a = ((Y * hRT) * sp[s].RW) * T;
-        b = (Y * cpR) * sp[s].RW;
-      }
-      bool placed = false;
-#pragma unroll
-      for (int l = 0; l < 6; ++l) {
-        if (!placed) {
-          if ((s >> l) & 1) {  // the right subtree at level l: join its pending left sibling
-            a = sh[l] + a;
-            b = sc[l] + b;
-          } else {  // a left subtree: pending until its sibling is complete
-            sh[l] = a;
-            sc[l] = b;
-            placed = true;
-          }
-        }
-      }
-      if (s == 63) {  // every level has joined: the totals
-        hm = a;
-        cpm = b;
-      }
-    }
-    const double dT = (h - hm) / cpm;
-    T = T + dT;
-    if (fabs(dT) <= 1e-10 * T) break;
-  }
-  return T;
-}
 
 template <int N, int R, int MODE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) eos_cell_kernel(EosParams P) {
@@ -96,12 +48,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) e
     const int i = P.lo0 + (int)(u % (unsigned)P.nx);
     const int j = P.lo1 + (int)((u / (unsigned)P.nx) % (unsigned)P.ny);
     const int k = P.lo2 + (int)(u / ((unsigned)P.nx * (unsigned)P.ny));
-    if constexpr (MODE == EOS_SET_T) {
-      const double rhoinv = 1.0 / P.rho.p[aoff(P.rho, i, j, k)];
-      const long offY = aoff(P.rY, i, j, k), oT = aoff(P.T, i, j, k);
-      P.T.p[oT] = hy2t_cell<N>(sp, P.rY.p + offY, P.rY.ns, rhoinv, (P.rH.p[aoff(P.rH, i, j, k)] * rhoinv) * 1.0e4,
-                               P.T.p[oT]);
-    } else if constexpr (MODE == EOS_FLOOR) {
+    if constexpr (MODE == EOS_FLOOR) {
       const long offY = aoff(P.rY, i, j, k);
       double rho = 0.0;
 #pragma unroll 4
@@ -137,6 +84,44 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) e
       }
       P.HR.p[aoff(P.HR, i, j, k)] = hr;
     }
+  }
+}
+
+// setTemperature with G lanes per cell in the rows layout (block_rates.h): the pairwise sums start
+// inside a lane and end in DPP adds. What bounds it is the latency of the iteration (a reciprocal,
+// two fourth-order polynomials per species, a division) for a box of tens of thousands of cells and
+// FP64 issue above. One thread per cell, the sums over a tree of pending partial sums, was slower at
+// every size (us per call, thread / rows): drm19 512 cells 66 / 26, 64000 71 / 32, 262144 97 / 59,
+// 884736 223 / 131; dodecane_lu 64000 91 / 50, 884736 378 / 351; LiDryer 262144 80 / 42.
+template <int N, int R, int G>
+__global__ void __launch_bounds__(256) set_temp_rows_kernel(EosParams P) {
+  using C = BlockCell<N, R, G>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  {
+    const BlobLayout BL = blob_layout(N, R, P.neff, P.ninc);
+    const uint4* srcb = reinterpret_cast<const uint4*>(P.blob + BL.off_sp);
+    uint4* dst = reinterpret_cast<uint4*>(smem);
+    for (int b = threadIdx.x; b < (int)(N * sizeof(SpRec)) / 16; b += blockDim.x) dst[b] = srcb[b];
+  }
+  __syncthreads();
+  const SpRec* sp = reinterpret_cast<const SpRec*>(smem);
+  const int lane = threadIdx.x % G;
+  const long stride = (long)gridDim.x * (blockDim.x / G);
+  for (long c = (long)blockIdx.x * (blockDim.x / G) + threadIdx.x / G; c < P.ncells; c += stride) {
+    const unsigned u = (unsigned)c;
+    const int i = P.lo0 + (int)(u % (unsigned)P.nx);
+    const int j = P.lo1 + (int)((u / (unsigned)P.nx) % (unsigned)P.ny);
+    const int k = P.lo2 + (int)(u / ((unsigned)P.nx * (unsigned)P.ny));
+    const double rhoinv = 1.0 / P.rho.p[aoff(P.rho, i, j, k)];
+    const long offY = aoff(P.rY, i, j, k), oT = aoff(P.T, i, j, k);
+    double Y[C::RPL];
+#pragma unroll
+    for (int s = 0; s < C::RPL; ++s) {
+      const int ii = C::row(lane, s);
+      Y[s] = ii < N ? P.rY.p[offY + (long)ii * P.rY.ns] * rhoinv : 0.0;
+    }
+    const double T = rows_hy2t<N, R, G>(sp, lane, Y, (P.rH.p[aoff(P.rH, i, j, k)] * rhoinv) * 1.0e4, P.T.p[oT]);
+    if (lane == 0) P.T.p[oT] = T;
   }
 }
 

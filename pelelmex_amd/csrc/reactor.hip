@@ -63,6 +63,7 @@ using EvalLaunch = hipError_t (*)(int mode, const unsigned char* blob, int blob_
 using Occ = hipError_t (*)(int* nb, int block, size_t shmem);
 using RateLaunch = hipError_t (*)(const prk::RateParams&, int blocks, int block, size_t shmem, hipStream_t);
 using BlockRateLaunch = hipError_t (*)(const prk::RateParams&, const prk::BlockTabs&, int cus, hipStream_t);
+using SetTempLaunch = hipError_t (*)(const prk::EosParams&, int cus, hipStream_t);
 using TrustLaunch = hipError_t (*)(const prk::TrustParams&, int blocks, int block, size_t shmem, hipStream_t);
 using FeatLaunch = hipError_t (*)(const prk::FeatParams&, hipStream_t);
 using PrepLaunch = hipError_t (*)(const prk::PrepParams&, int blocks, int block, size_t shmem, hipStream_t);
@@ -110,6 +111,14 @@ hipError_t rates_block_t(const prk::RateParams& P, const prk::BlockTabs& tab, in
 }
 
 template <int N, int R, int G>
+hipError_t set_temp_t(const prk::EosParams& P, int cus, hipStream_t st) {
+  const long want = (P.ncells + 256 / G - 1) / (256 / G), cap = 16L * cus;
+  hipLaunchKernelGGL((prk::set_temp_rows_kernel<N, R, G>), dim3((unsigned)(want < cap ? want : cap)), dim3(256),
+                     N * sizeof(prk::SpRec), st, P);
+  return hipGetLastError();
+}
+
+template <int N, int R, int G>
 hipError_t trust_t(const prk::TrustParams& P, int blocks, int block, size_t shmem, hipStream_t st) {
   hipLaunchKernelGGL((prk::trust_kernel<N, R, G>), dim3(blocks), dim3(block), shmem, st, P);
   return hipGetLastError();
@@ -123,9 +132,7 @@ hipError_t prep_t(const prk::PrepParams& P, int blocks, int block, size_t shmem,
 
 template <int N, int R, int G>
 hipError_t eos_t(int mode, const prk::EosParams& P, int blocks, int block, size_t shmem, hipStream_t st) {
-  if (mode == prk::EOS_SET_T)
-    hipLaunchKernelGGL((prk::eos_cell_kernel<N, R, prk::EOS_SET_T>), dim3(blocks), dim3(block), shmem, st, P);
-  else if (mode == prk::EOS_FLOOR)
+  if (mode == prk::EOS_FLOOR)
     hipLaunchKernelGGL((prk::eos_cell_kernel<N, R, prk::EOS_FLOOR>), dim3(blocks), dim3(block), shmem, st, P);
   else
     hipLaunchKernelGGL((prk::eos_cell_kernel<N, R, prk::EOS_HEAT_RELEASE>), dim3(blocks), dim3(block), shmem, st, P);
@@ -222,11 +229,12 @@ struct BlockOps {
   const char* mech;
   int waves, nchunk;
   BlockRateLaunch rates;
+  SetTempLaunch set_temp;
 };
 
 #define PR_BLOCK_OPS(NAME, NS, NR) \
   {NAME, block_lanes(NS + 1), prk::BlockCell<NS, NR, block_lanes(NS + 1)>::NCHUNK, \
-   &rates_block_t<NS, NR, block_lanes(NS + 1)>}
+   &rates_block_t<NS, NR, block_lanes(NS + 1)>, &set_temp_t<NS, NR, block_lanes(NS + 1)>}
 
 const BlockOps kBlockOps[] = {
     PR_BLOCK_OPS("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR),
@@ -1969,7 +1977,8 @@ static int eos_launch(pr_handle* h, int mode, const int lo[3], const int hi[3], 
   const long cap = 8L * dev_cus;
   const int blocks = (int)(want < cap ? want : cap);
   hipStream_t st = (hipStream_t)stream;
-  HIPCHK(h->var->eos(mode, P, blocks, block, shmem, st));
+  if (mode == prk::EOS_SET_T) HIPCHK(h->blk->set_temp(P, dev_cus, st));
+  else HIPCHK(h->var->eos(mode, P, blocks, block, shmem, st));
   HIPCHK(hipStreamSynchronize(st));
   return 0;
 }

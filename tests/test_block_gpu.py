@@ -71,3 +71,23 @@ def test_react_variant_by_size(gpu, mech, cells, lanes):
     for k in range(4):
         _bits(("rY", "T", "rH", "FC")[k], out[0][k], out[1][k])
     assert out[0][4] == out[1][4] and all(out[0][5][k] == out[1][5][k] for k in ("nst", "nfe", "nje", "nsetups", "nni"))
+
+
+# 64 cells per block of setTemperature (32 with 8 lanes per cell): one cell, all but one, one more
+@pytest.mark.parametrize("mech,cells", [("drm19", 1), ("drm19", 63), ("drm19", 64), ("drm19", 65), ("LiDryer", 17),
+                                        ("dodecane_lu", 1), ("dodecane_lu", 31), ("dodecane_lu", 33), ("syn53", 100)])
+def test_set_temperature_rows(gpu, mech, cells):
+    import torch
+    from oracle import pyoracle as po
+    from pelelmex_amd.reactor import Reactor
+    box = BOXES[mech](nx=cells, ny=1, nz=1)
+    m = po.Mech(mech)
+    rY, rH = box["rY"] * 1e3, box["rH"] * 0.1
+    rho, T0 = rY.sum(0), box["T"] + 25.0 * np.sin(np.arange(cells))
+    r = Reactor.create("ReactorCvode", mech, KEYS)
+    r.init(2, 1)
+    dev = lambda a, *shape: torch.as_tensor(np.ascontiguousarray(a)).reshape(*shape).to(gpu).contiguous()
+    T = dev(T0, 1, 1, cells).clone()
+    r.set_temperature(dev(rho, 1, 1, cells), dev(rY, m.nsp, 1, 1, cells), dev(rH, 1, 1, cells), T)
+    r.close()
+    _bits("T", T.cpu().numpy().reshape(-1), m.set_temperature(rho, rY, rH, T0))
