@@ -1163,7 +1163,7 @@ __device__ __forceinline__ bool lu_factor(const Smem<N, R>& S, int lane, double 
 // step k in lane k.
 template <int N, int R, int G>
 constexpr bool lu_pivot_order() {
-  return (G == 32 && Cell<N, R, G>::RPL == 1) || Cell<N, R, G>::lu_global;
+  return (G == 32 && Cell<N, R, G>::RPL == 1) || G == 64;
 }
 
 template <int N, int R, int G>
@@ -1210,23 +1210,6 @@ __device__ __forceinline__ void lu_solve(const Smem<N, R>& S, int lane, const do
                                          int permv, double (&b)[Cell<N, R, G>::RPL], double (&x)[Cell<N, R, G>::RPL]) {
   constexpr int RPL = Cell<N, R, G>::RPL;
   constexpr int n = N + 1;
-  if constexpr (G == 64 && !lu_pivot_order<N, R, G>()) {
-#pragma unroll
-    for (int k = 0; k < n; ++k) {
-      const int p = __builtin_amdgcn_readlane(permv, k);
-      const double yk = rlane_d(b[0], p);
-      if (pst[0] > k) b[0] = fma(-lu[0][k], yk, b[0]);
-    }
-    x[0] = 0.0;
-#pragma unroll
-    for (int k = n - 1; k >= 0; --k) {
-      const int p = __builtin_amdgcn_readlane(permv, k);
-      const double xk = rlane_d(b[0], p) * rlane_d(rinv[0], p);
-      if (pst[0] >= 0 && pst[0] < k) b[0] = fma(-lu[0][k], xk, b[0]);
-      if (lane == k) x[0] = xk;
-    }
-    return;
-  }
   if constexpr (lu_pivot_order<N, R, G>()) {
     // lane k holds the row pivoted at step k (pst = k); its right-hand side entry is b[p_k].
     // Step k's value comes from lane k of the group through the LDS crossbar (ds_bpermute, the
@@ -1239,12 +1222,12 @@ __device__ __forceinline__ void lu_solve(const Smem<N, R>& S, int lane, const do
         (lane < n) ? 1.0 / S.LU[lane * n + lane] : 0.0;  // the diagonal entry in either layout
 #pragma unroll
     for (int k = 0; k < n; ++k) {
-      const double yk = bperm_d(v, base + 4 * k);
+      const double yk = Cell<N, R, G>::js_lds ? rlane_d(v, k) : bperm_d(v, base + 4 * k);
       if (ol > k && ol < n) v = fma(-lu[0][k], yk, v);
     }
 #pragma unroll
     for (int k = n - 1; k >= 1; --k) {
-      const double xk = bperm_d(v * rdiag, base + 4 * k);
+      const double xk = Cell<N, R, G>::js_lds ? rlane_d(v * rdiag, k) : bperm_d(v * rdiag, base + 4 * k);
       if (ol < k) v = fma(-lu[0][k], xk, v);
     }
     x[0] = v * rdiag;  // lane k's v is final from step k on: x_k = v_k / pivot_k
