@@ -255,25 +255,39 @@ const Variant* find_variant(const char* mech, int G, int W = 0) {
   return nullptr;
 }
 
-// Small launches: the launch lasts as long as its stiffest cell's integration (four times the mean's
-// right-hand sides) whatever is idle, so a cell gets more lanes (fewer passes over the reactions) and
-// shares its wavefront with fewer others (no waiting for their Jacobians and factorizations). A rule
-// holds for launches of up to max_cells cells when no key chooses a variant; all variants give the
-// same bits. The lines lie where the wider variant stops winning when cells come in natural order (a
-// first call); with the cost order they would lie higher. Measured, ms per call, natural order /
-// cost order: drm19, 64 lanes against 32: 512 cells 7.1 / 7.2 against 11.8 / 10.9, 4096 9.5 / 7.9
-// against 11.8 / 11.7, 5832 11.5 / 7.7 against 12.5 / 11.9, 8000 13.8 / 8.1 against 13.1 / 12.5.
-// LiDryer, 64 / 32 / 16 lanes: 512 cells 1.63 / 1.74 / 2.85 natural, 1.63 / 1.78 / 2.28 ordered;
-// 1728 1.91 / 1.85 / 2.79 and 1.70 / 1.92 / 2.4; 5832 3.81 / 2.40 / 2.93 natural; 8000 4.8 / 3.0 /
-// 2.97 and 4.0 / 2.2 / 2.65. 54 components run 64 lanes at every size.
+// The variant of a launch of up to max_cells cells when no key chooses one; all variants give the same
+// bits. A small launch lasts as long as its stiffest cell's integration (four times the mean's
+// right-hand sides) whatever is idle: a cell gets more lanes (fewer passes over the reactions) and
+// shares its wavefront with fewer others (no waiting for their Jacobians and factorizations), and
+// its kernel more registers. A large one gets more resident cells, spills or not. The lines lie
+// where the smaller side's variant stops winning when cells come in natural order (a first call);
+// with the cost order they would lie higher. Measured, ms per call, natural / cost order:
+//  drm19, 64 lanes against 32: 512 cells 7.1 / 7.2 against 11.8 / 10.9, 4096 9.5 / 7.9 against
+//   11.8 / 11.7, 5832 11.5 / 7.7 against 12.5 / 11.9, 8000 13.8 / 8.1 against 13.1 / 12.5.
+//  LiDryer, 64 / 32 / 16 lanes: 512 cells 1.63 / 1.74 / 2.85 natural, 1.63 / 1.78 / 2.28 ordered;
+//   1728 1.91 / 1.85 / 2.79 and 1.70 / 1.92 / 2.4; 5832 3.81 / 2.40 / 2.93 natural; 8000 4.8 / 3.0 /
+//   2.97 and 4.0 / 2.2 / 2.65. 16 lanes, 3 waves against 4: 13824 3.84 / 2.71 against 4.19 / 2.89,
+//   27000 6.26 / 4.06 against 6.11 / 4.21, 32768 6.87 / 4.73 against 6.81 / 4.51, 262144 38.2 / 35.9
+//   against 35.7 / 32.5.
+//  dodecane_lu, 2 waves against 3: 512 cells 36.2 / 31.4 against 37.7 / 34.5, 5832 53.8 / 36.5 against
+//   52.5 / 39.0, 8000 66.0 / 44.6 against 62.2 / 38.9, 32768 200 / 175 against 174 / 148. syn53: 4096
+//   29.5 / 20.8 against 28.0 / 21.9, 13824 62.1 / 48.7 against 57.2 / 42.2.
 struct SizeRule {
   long max_cells;
   Variant v;
 };
+constexpr long kAnySize = 1L << 62;
 const SizeRule kSizeRules[] = {  // per mechanism in ascending order
     {2048, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 64, 2)},
     {7168, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 32, 3)},
+    {28672, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 3)},
+    {kAnySize, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 4)},
     {6144, PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 64, 2)},
+    {kAnySize, PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 32, 4)},
+    {6144, PR_VARIANT("syn53", PR_SYN53_NSP, PR_SYN53_NR, 64, 2)},
+    {kAnySize, PR_VARIANT("syn53", PR_SYN53_NSP, PR_SYN53_NR, 64, 3)},
+    {6144, PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 2)},
+    {kAnySize, PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 3)},
 };
 
 std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
@@ -848,16 +862,18 @@ static int bdf_block(const pr_handle* h, const Variant* v) {
   return 64;
 }
 
-// BDF kernel of a launch of up to work cells: the handle's variant, unless the keys leave the
-// choice open and the launch is small (kSizeRules). All variants give the same bits.
-static const Variant* bdf_variant(const pr_handle* h, long work, int* block) {
+// BDF kernel of a launch of up to work cells: the handle's variant when a key chooses one, else by
+// size. slots: bytes of global slots that smaller launches of the handle may need.
+static const Variant* bdf_variant(const pr_handle* h, long work, int* block, size_t* slots) {
   const Keys& K = h->keys;
   const Variant* v = h->var;
+  *slots = 0;
   if (!K.lanes_per_cell && !K.waves && !K.block && !K.autotune)
     for (const SizeRule& r : kSizeRules)
-      if (std::strcmp(r.v.mech, h->mech->name) == 0 && work <= r.max_cells) {
+      if (std::strcmp(r.v.mech, h->mech->name) == 0) {
         v = &r.v;
-        break;
+        if (work <= r.max_cells) break;
+        *slots = std::max(*slots, (size_t)(r.max_cells + 256 * r.v.waves / r.v.G) * (size_t)r.v.slot);
       }
   *block = bdf_block(h, v);
   return v;
@@ -894,7 +910,8 @@ static prk::Arr to_arr(const pr_array4* a) {
 static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t st, double* gscr = nullptr,
                       size_t gscr_cap = 0) {
   int block = 0;
-  const Variant* v = bdf_variant(h, work_max, &block);
+  size_t smaller = 0;
+  const Variant* v = bdf_variant(h, work_max, &block, &smaller);
   const int G = v->G;
   if (block > 256 * v->waves)
     return fail(PR_ERR_KEY, "hipbdf.block " + std::to_string(block) + " exceeds " + std::to_string(256 * v->waves) +
@@ -917,13 +934,8 @@ static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t 
   if (gscr) {
     P.gscr = gscr;
   } else {
-    size_t need = (size_t)blocks * (size_t)(block / G) * (size_t)v->slot;
-    // a smaller launch of this handle may take another variant; it finds its slots allocated, as a
-    // captured one has to
-    if (v == h->var)
-      for (const SizeRule& r : kSizeRules)
-        if (std::strcmp(r.v.mech, h->mech->name) == 0)
-          need = std::max(need, (size_t)(r.max_cells + 256 * r.v.waves / r.v.G) * (size_t)r.v.slot);
+    // a smaller launch may take another variant; it finds its slots allocated, as a captured one has to
+    const size_t need = std::max(smaller, (size_t)blocks * (size_t)(block / G) * (size_t)v->slot);
     int rc = ensure_gscr(h, need);
     if (rc) return rc;
     P.gscr = h->d_gscr;

@@ -50,16 +50,20 @@ def test_reaction_rates_64_cells_per_block(gpu, mech, dims):
     _bits("rYdot", out.cpu().numpy().reshape(m.nsp, nc), ref)
 
 
-@pytest.mark.parametrize("mech,cells,lanes", [("LiDryer", 1, 64), ("LiDryer", 2048, 64), ("LiDryer", 2049, 32),
-                                              ("LiDryer", 7168, 32), ("LiDryer", 7169, 16), ("drm19", 1, 64),
-                                              ("drm19", 6144, 64), ("drm19", 6145, 32)])
-def test_react_variant_by_size(gpu, mech, cells, lanes):
+LARGE = {"LiDryer": (16, 3), "drm19": (32, 4), "dodecane_lu": (64, 2), "syn53": (64, 2)}
+
+
+@pytest.mark.parametrize("mech,cells,lanes,waves", [
+    ("LiDryer", 1, 64, 2), ("LiDryer", 2048, 64, 2), ("LiDryer", 2049, 32, 3), ("LiDryer", 7168, 32, 3),
+    ("LiDryer", 7169, 16, 3), ("LiDryer", 28673, 16, 4), ("drm19", 1, 64, 2), ("drm19", 6144, 64, 2),
+    ("drm19", 6145, 32, 4), ("dodecane_lu", 6144, 64, 2), ("dodecane_lu", 6145, 64, 3), ("syn53", 6145, 64, 3)])
+def test_react_variant_by_size(gpu, mech, cells, lanes, waves):
     """A launch's variant follows its cell count unless a key chooses one; the bits do not."""
     import torch
     from pelelmex_amd.reactor import Reactor, box_tensors
     box = BOXES[mech](nx=cells, ny=1, nz=1)
     out = []
-    for keys in (KEYS, dict(KEYS, **{"hipbdf.lanes_per_cell": 16 if mech == "LiDryer" else 32})):
+    for keys in (KEYS, dict(KEYS, **{"hipbdf.lanes_per_cell": LARGE[mech][0], "hipbdf.waves_per_simd": LARGE[mech][1]})):
         r = Reactor.create("ReactorCvode", mech, dict(keys, **{"cvode.max_order": 4}))
         r.init(2, 1)
         t = box_tensors(box, gpu)
@@ -67,7 +71,7 @@ def test_react_variant_by_size(gpu, mech, cells, lanes):
         torch.cuda.synchronize()
         out.append([t[k].cpu().numpy() for k in ("rY", "T", "rH", "FC")] + [nfail, r.stats()])
         r.close()
-    assert out[0][5]["lanes_per_cell"] == lanes
+    assert (out[0][5]["lanes_per_cell"], out[0][5]["waves_per_simd"]) == (lanes, waves)
     for k in range(4):
         _bits(("rY", "T", "rH", "FC")[k], out[0][k], out[1][k])
     assert out[0][4] == out[1][4] and all(out[0][5][k] == out[1][5][k] for k in ("nst", "nfe", "nje", "nsetups", "nni"))
