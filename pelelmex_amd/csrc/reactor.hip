@@ -12,6 +12,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <map>
 #include <mutex>
 #include <sstream>
 #include <string>
@@ -533,6 +534,39 @@ std::vector<unsigned char> pack_jac_tabs(const pr_mech_t* m, const std::vector<u
   return out;
 }
 
+// The device tables of a mechanism as one image, built once per process: blob, block tables,
+// Jacobian tables, each section from a multiple of 256 bytes.
+struct MechImage {
+  std::vector<unsigned char> bytes;
+  int blob_bytes = 0, njac = 0;
+  size_t tabs[4], jtabs[3];  // offsets
+};
+
+const MechImage& mech_image(const pr_mech_t* m, const BlockOps* blk) {
+  static std::mutex mu;
+  static std::map<const pr_mech_t*, MechImage> images;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = images.find(m);
+  if (it != images.end()) return it->second;
+  MechImage im;
+  const std::vector<unsigned char> blob = pack_blob(m);
+  const std::vector<unsigned char> tabs = pack_block_tabs(m, blob, blk->waves, blk->nchunk, im.tabs);
+  const std::vector<unsigned char> jtabs = pack_jac_tabs(m, blob, im.jtabs, &im.njac);
+  im.blob_bytes = (int)blob.size();
+  auto put = [&](const std::vector<unsigned char>& v) {
+    const size_t at = im.bytes.size();
+    im.bytes.insert(im.bytes.end(), v.begin(), v.end());
+    im.bytes.resize((im.bytes.size() + 255) / 256 * 256, 0);
+    return at;
+  };
+  put(blob);
+  const size_t t = put(tabs);
+  for (size_t& o : im.tabs) o += t;
+  const size_t j = put(jtabs);
+  for (size_t& o : im.jtabs) o += j;
+  return images.emplace(m, std::move(im)).first->second;
+}
+
 struct Keys {
   double rtol = 1e-10, atol = 1e-10;
   int max_order = 2, max_substeps = 10000;
@@ -687,13 +721,11 @@ struct pr_handle {
   Keys keys;
   int device = 0;
   int block = 128;
-  unsigned char* d_blob = nullptr;
+  unsigned char* d_blob = nullptr;  // one allocation: the mechanism's image, d_atolv, d_counters
   int blob_bytes = 0;
   const BlockOps* blk = nullptr;
-  prk::BlockTabs tabs{};       // device tables of the block kernels, one allocation
-  void* d_tabs = nullptr;
-  prk::JacTabs jtabs{};        // device tables of the Jacobian, one allocation
-  void* d_jtabs = nullptr;
+  prk::BlockTabs tabs{};       // device tables of the block kernels
+  prk::JacTabs jtabs{};        // and of the Jacobian
   double* d_atolv = nullptr;
   void* d_counters = nullptr;  // two regions of 128 B: queue (4 B), nfail (4 B), stats (8 x 8 B at +64)
   double* d_gscr = nullptr;    // per-group global scratch slots
@@ -768,49 +800,44 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
     delete h;
     return rc;
   }
-  std::vector<unsigned char> blob = pack_blob(m);
-  h->blob_bytes = (int)blob.size();
+  h->blk = find_block_ops(m->name);
+  const MechImage& im = mech_image(m, h->blk);
+  h->blob_bytes = im.blob_bytes;
   {
     // the gather's block sums are held in the group's 5 N species doubles of LDS
     const prk::BlobLayout L = prk::blob_layout(m->nsp, m->nr, m->neff, m->ninc);
-    const int nb = reinterpret_cast<const int*>(blob.data() + L.off_kblk)[m->nsp];
+    const int nb = reinterpret_cast<const int*>(im.bytes.data() + L.off_kblk)[m->nsp];
     if (nb > 5 * m->nsp) {
       delete h;
       return fail(PR_ERR_UNSUPPORTED, "mechanism has more production-rate gather blocks than 5 per species");
     }
   }
-  // per-component absolute tolerances: ode.atol everywhere until set_typ_vals_ode scales them
-  // (the kernels always read this array, so a captured graph sees later typical values)
-  size_t toff[4];
-  h->blk = find_block_ops(m->name);
-  const std::vector<unsigned char> tabs = pack_block_tabs(m, blob, h->blk->waves, h->blk->nchunk, toff);
-  size_t joff[3];
-  const std::vector<unsigned char> jtabs = pack_jac_tabs(m, blob, joff, &h->jtabs.nentry);
+  // One allocation: the mechanism's image, the per-component absolute tolerances (ode.atol everywhere
+  // until set_typ_vals_ode scales them; the kernels always read this array, so a captured graph sees
+  // later typical values) and the counters.
+  std::vector<unsigned char> init = im.bytes;
   const std::vector<double> atol0((size_t)m->nsp + 1, K.atol);
-  if (hipMalloc(&h->d_blob, blob.size()) != hipSuccess || hipMalloc(&h->d_counters, 256) != hipSuccess ||
-      hipMalloc(&h->d_tabs, tabs.size()) != hipSuccess || hipMalloc(&h->d_jtabs, jtabs.size()) != hipSuccess ||
-      hipMemcpy(h->d_jtabs, jtabs.data(), jtabs.size(), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(h->d_tabs, tabs.data(), tabs.size(), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMalloc(&h->d_atolv, sizeof(double) * (m->nsp + 1)) != hipSuccess ||
-      hipMemcpy(h->d_atolv, atol0.data(), sizeof(double) * atol0.size(), hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(h->d_blob, blob.data(), blob.size(), hipMemcpyHostToDevice) != hipSuccess ||
+  const size_t at_atol = init.size();
+  init.resize(at_atol + (sizeof(double) * atol0.size() + 255) / 256 * 256 + 256, 0);
+  std::memcpy(init.data() + at_atol, atol0.data(), sizeof(double) * atol0.size());
+  if (hipMalloc(&h->d_blob, init.size()) != hipSuccess ||
+      hipMemcpy(h->d_blob, init.data(), init.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess ||
       hipEventCreate(&h->ev2) != hipSuccess || hipEventCreate(&h->ev3) != hipSuccess) {
     pr_destroy(h);
     return fail(PR_ERR_HIP, "device allocation failed");
   }
-  {
-    auto* t = static_cast<unsigned char*>(h->d_tabs);
-    h->tabs.rx = reinterpret_cast<const prk::RxRec*>(t + toff[0]);
-    h->tabs.rx_range = reinterpret_cast<const int32_t*>(t + toff[1]);
-    h->tabs.piece = reinterpret_cast<const prk::GatherPiece*>(t + toff[2]);
-    h->tabs.piece_range = reinterpret_cast<const int32_t*>(t + toff[3]);
-    h->tabs.nchunk = h->blk->nchunk;
-    auto* j = static_cast<unsigned char*>(h->d_jtabs);
-    h->jtabs.term = reinterpret_cast<const prk::JacTerm*>(j + joff[0]);
-    h->jtabs.entry = reinterpret_cast<const prk::JacEntry*>(j + joff[1]);
-    h->jtabs.slice = reinterpret_cast<const int32_t*>(j + joff[2]);
-  }
+  h->d_atolv = reinterpret_cast<double*>(h->d_blob + at_atol);
+  h->d_counters = h->d_blob + init.size() - 256;
+  h->tabs.rx = reinterpret_cast<const prk::RxRec*>(h->d_blob + im.tabs[0]);
+  h->tabs.rx_range = reinterpret_cast<const int32_t*>(h->d_blob + im.tabs[1]);
+  h->tabs.piece = reinterpret_cast<const prk::GatherPiece*>(h->d_blob + im.tabs[2]);
+  h->tabs.piece_range = reinterpret_cast<const int32_t*>(h->d_blob + im.tabs[3]);
+  h->tabs.nchunk = h->blk->nchunk;
+  h->jtabs.term = reinterpret_cast<const prk::JacTerm*>(h->d_blob + im.jtabs[0]);
+  h->jtabs.entry = reinterpret_cast<const prk::JacEntry*>(h->d_blob + im.jtabs[1]);
+  h->jtabs.slice = reinterpret_cast<const int32_t*>(h->d_blob + im.jtabs[2]);
+  h->jtabs.nentry = im.njac;
   *out = h;
   return 0;
 }
@@ -2538,10 +2565,6 @@ int pr_get_stats(const pr_handle* h, pr_stats* out) {
 void pr_destroy(pr_handle* h) {
   if (!h) return;
   if (h->d_blob) (void)hipFree(h->d_blob);
-  if (h->d_counters) (void)hipFree(h->d_counters);
-  if (h->d_tabs) (void)hipFree(h->d_tabs);
-  if (h->d_jtabs) (void)hipFree(h->d_jtabs);
-  if (h->d_atolv) (void)hipFree(h->d_atolv);
   if (h->d_gscr) (void)hipFree(h->d_gscr);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
