@@ -80,11 +80,12 @@ template <int N, int R, int G>
 hipError_t eval_t(int mode, const unsigned char* blob, int blob_bytes, int neff, int ninc, long ncells, const double* y,
                   const double* rYsrc, const double* rhoh0, const double* rhohsrc, double t, double* out, double* gscr,
                   const prk::JacTabs& jt, int blocks, int block, size_t shmem, hipStream_t st) {
+  const size_t jac = sizeof(double) * (size_t)(block / G) * (size_t)prk::eval_jac_doubles<N, R, G>();
   if (mode == 0)
     hipLaunchKernelGGL((prk::eval_kernel<N, R, G, 0>), dim3(blocks), dim3(block), shmem, st, blob, blob_bytes, neff,
                        ninc, ncells, y, rYsrc, rhoh0, rhohsrc, t, out, gscr, jt);
   else
-    hipLaunchKernelGGL((prk::eval_kernel<N, R, G, 1>), dim3(blocks), dim3(block), shmem, st, blob, blob_bytes, neff,
+    hipLaunchKernelGGL((prk::eval_kernel<N, R, G, 1>), dim3(blocks), dim3(block), shmem + jac, st, blob, blob_bytes, neff,
                        ninc, ncells, y, rYsrc, rhoh0, rhohsrc, t, out, gscr, jt);
   return hipGetLastError();
 }

@@ -95,3 +95,26 @@ def test_set_temperature_rows(gpu, mech, cells):
     r.set_temperature(dev(rho, 1, 1, cells), dev(rY, m.nsp, 1, 1, cells), dev(rH, 1, 1, cells), T)
     r.close()
     _bits("T", T.cpu().numpy().reshape(-1), m.set_temperature(rho, rY, rH, T0))
+
+
+# a block writes its cells' Jacobians together: one cell, a part of a block, whole blocks and one more,
+# through the LU area (8, 16 lanes), extra LDS (32) and straight from the group (64)
+@pytest.mark.parametrize("mech,lanes", [("LiDryer", 8), ("LiDryer", 16), ("drm19", 16), ("drm19", 32), ("drm19", 64),
+                                        ("dodecane_lu", 64)])
+@pytest.mark.parametrize("cells", [1, 7, 33])
+def test_jacobians_by_block(gpu, mech, lanes, cells):
+    import torch
+    from oracle import pyoracle as po
+    from pelelmex_amd.reactor import Reactor
+    box = BOXES[mech](nx=cells, ny=1, nz=1)
+    m = po.Mech(mech)
+    y = np.vstack([box["rY"], box["T"][None, :]])
+    ref = np.zeros((m.nsp + 1, m.nsp + 1, cells))
+    for c in range(cells):
+        ref[:, :, c] = m.jac(m.cell(box["rH"][c], box["rHsrc"][c], box["rYsrc"][:, c]), 0.0, y[:, c])
+    r = Reactor.create("ReactorCvode", mech, dict(KEYS, **{"hipbdf.lanes_per_cell": lanes}))
+    r.init(2, 1)
+    dev = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64).to(gpu)
+    J = r.jac_batch(dev(y), dev(box["rYsrc"]), dev(box["rHsrc"])).cpu().numpy()
+    r.close()
+    _bits("jac", J, ref)
