@@ -290,28 +290,54 @@ __global__ void gelu_bwd_kernel(long rows, int cols, const float* dA, long lda, 
   if (dZ) dZ[r * ldd + c] = g;
 }
 
-// db[c] = sum over rows of d[r, c]: 16 columns per block, 64 row groups of 16 lanes, each summing
-// its rows (r, r + 64, ..) with eight loads in flight, then a pairwise tree over the groups. 16
-// columns and not 64 per block: a layer of 256 then has 16 blocks instead of 4 (4096 rows: 240 us
-// with 4 row groups and 64 columns, 9 us now).
-constexpr int kSumCols = 16;
-__global__ void __launch_bounds__(1024) col_sum_kernel(long rows, int cols, const float* d, long ld, float* out,
-                                                       int accumulate) {
-  __shared__ float part[64][kSumCols];
-  const int cl = threadIdx.x % kSumCols, rg = threadIdx.x / kSumCols;
+// db[c] = sum over rows of d[r, c]: four partial sums of the rows r, r + 4, .., each in row order (the
+// first Adam step divides a bias gradient by its own magnitude, so its rounding is part of the
+// result), then (0 + 1) + (2 + 3). 16 columns per block; 512 threads stage 512 rows in LDS, the next
+// tile's loads in flight while one wavefront adds. What bounds it is that wavefront's chain of
+// additions: 4096 rows of 256 columns 240 us with the adding threads reading memory themselves (64
+// columns per block), 16 us now (9 us with a tree over 64 partial sums, whose rounding shifted the
+// first steps of biases with gradients near Adam's epsilon).
+constexpr int kSumCols = 16, kSumRows = 512;
+__global__ void __launch_bounds__(512) col_sum_kernel(long rows, int cols, const float* d, long ld, float* out,
+                                                      int accumulate) {
+  __shared__ float tile[kSumRows * kSumCols];
+  __shared__ float part[4][kSumCols];
+  const int t = threadIdx.x, cl = t % kSumCols;
   const int c = blockIdx.x * kSumCols + cl;
+  constexpr int NL = kSumCols;  // rows a thread stages: t / 16 + 32 j
+  float v[NL];
+  auto load = [&](long r0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const long r = r0 + t / kSumCols + (long)(kSumRows / NL) * j;
+      v[j] = (c < cols && r < rows) ? d[r * ld + c] : 0.f;
+    }
+  };
+  const int rg = t / kSumCols;  // partial sum of the adding threads (t < 64)
   float s = 0.f;
-  if (c < cols) {
-#pragma unroll 8
-    for (long r = rg; r < rows; r += 64) s += d[r * ld + c];
-  }
-  part[rg][cl] = s;
-  __syncthreads();
-  for (int w = 32; w > 0; w >>= 1) {
-    if (rg < w) part[rg][cl] += part[rg + w][cl];
+  load(0);
+  for (long r0 = 0; r0 < rows; r0 += kSumRows) {
+#pragma unroll
+    for (int j = 0; j < NL; ++j) tile[t + kSumRows * j] = v[j];
+    __syncthreads();
+    if (r0 + kSumRows < rows) load(r0 + kSumRows);
+    if (t < 4 * kSumCols) {
+      const int m = (int)(rows - r0 < kSumRows ? rows - r0 : kSumRows);
+      if (m == kSumRows) {
+#pragma unroll 32
+        for (int i = 0; i < kSumRows / 4; ++i) s += tile[(4 * i + rg) * kSumCols + cl];
+      } else {
+        for (int r = rg; r < m; r += 4) s += tile[r * kSumCols + cl];
+      }
+    }
     __syncthreads();
   }
-  if (rg == 0 && c < cols) out[c] = accumulate ? out[c] + part[0][cl] : part[0][cl];
+  if (t < 4 * kSumCols) part[rg][cl] = s;
+  __syncthreads();
+  if (t < kSumCols && c < cols) {
+    const float w = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
+    out[c] = accumulate ? out[c] + w : w;
+  }
 }
 
 // Mean-squared error over the first `cols` outputs: dY = 2 (Y - T) / (rows cols) (fp32, row

@@ -2520,7 +2520,7 @@ int pr_mlp_gelu_backward(int64_t rows, int cols, const float* dA, int64_t lda, c
 
 int pr_mlp_column_sum(int64_t rows, int cols, const float* d, int64_t ld, float* out, int accumulate, void* stream) {
   if (rows < 0 || cols < 1 || !d || !out) return fail(PR_ERR_ARG, "bad argument");
-  hipLaunchKernelGGL(prk::col_sum_kernel, dim3((unsigned)((cols + prk::kSumCols - 1) / prk::kSumCols)), dim3(1024), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL(prk::col_sum_kernel, dim3((unsigned)((cols + prk::kSumCols - 1) / prk::kSumCols)), dim3(512), 0, (hipStream_t)stream,
                      (long)rows, cols, d, (long)ld, out, accumulate);
   HIPCHK(hipGetLastError());
   return 0;
