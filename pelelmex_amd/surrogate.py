@@ -62,12 +62,44 @@ class MLP:
 
     def _init_state(self):
         import torch
-        self.Wb = [w.to(torch.bfloat16) for w in self.W]
-        self.gW = [torch.zeros_like(w) for w in self.W]
-        self.gb = [torch.zeros_like(b) for b in self.b]
-        self.m = [torch.zeros_like(p) for p in self.W + self.b]
-        self.v = [torch.zeros_like(p) for p in self.W + self.b]
+        # Parameters, gradients and Adam's moments each in one buffer, weights first, every tensor from
+        # a multiple of 64 elements; the lists hold views. Adam is then two launches, not two a layer.
+        params = self.W + self.b
+        offs, end = [], 0
+        for p in params:
+            offs.append(end)
+            end += (p.numel() + 63) // 64 * 64
+        self._nW = offs[len(self.W)]
+        self._flat = {k: torch.zeros(end, dtype=torch.float32, device=self.device) for k in "pgmv"}
+        self._flat["pb"] = torch.zeros(self._nW, dtype=torch.bfloat16, device=self.device)
+
+        def views(buf, like):
+            return [buf[o:o + p.numel()].view(p.shape) for o, p in zip(offs, like)]
+
+        new = views(self._flat["p"], params)
+        for q, p in zip(new, params):
+            q.copy_(p)
+        n = len(self.W)
+        self.W, self.b = new[:n], new[n:]
+        g = views(self._flat["g"], params)
+        self.gW, self.gb = g[:n], g[n:]
+        self.m, self.v = views(self._flat["m"], params), views(self._flat["v"], params)
+        self.Wb = views(self._flat["pb"], self.W)
+        for w, wb in zip(self.W, self.Wb):
+            wb.copy_(w)
         self.step = 0
+
+    def _in_place(self):
+        """Whether the lists still hold the views of the common buffers (a caller may put tensors of
+        its own into them)."""
+        f = self._flat
+        for k, ts in (("p", self.W + self.b), ("g", self.gW + self.gb), ("m", self.m), ("v", self.v), ("pb", self.Wb)):
+            at, size = f[k].data_ptr(), f[k].element_size()
+            for t in ts:
+                if t.data_ptr() != at or not t.is_contiguous():
+                    return False
+                at += (t.numel() + 63) // 64 * 64 * size
+        return True
 
     @property
     def nlayers(self):
@@ -130,7 +162,12 @@ class MLP:
         params = self.W + self.b
         grads = self.gW + self.gb
         bf = self.Wb + [None] * len(self.b)
-        for p, g, m, v, pb in zip(params, grads, self.m, self.v, bf):
+        parts = zip(params, grads, self.m, self.v, bf)
+        if self._in_place():
+            f, k = self._flat, self._nW
+            parts = [(f["p"][:k], f["g"][:k], f["m"][:k], f["v"][:k], f["pb"]),
+                     (f["p"][k:], f["g"][k:], f["m"][k:], f["v"][k:], None)]
+        for p, g, m, v, pb in parts:
             _chk(lib().pr_mlp_adam(p.numel(), _ptr(p), _ptr(g), _ptr(m), _ptr(v), _ptr(pb), lr, b1, b2, eps,
                                    self.step, _stream()), "pr_mlp_adam")
 
