@@ -867,7 +867,7 @@ __device__ __forceinline__ void rate_rhoY_eval(const Smem<N, R>& S, int lane, co
 // Every lane sums whole entries (JacTabs), in the order of the species' incidence list: a row per
 // lane instead left the lane of the longest list (84 of dodecane_lu's 918 entries) adding into its
 // row one dependent read-modify-write after another. What bounds it now is the rate pass; 8192
-// drm19 Jacobians 247 -> 97 us, and the react of 64^3 cells 122.4 -> 116.9 ms.
+// drm19 right-hand sides and Jacobians 292 -> 142 us, the react of 64^3 cells 122.4 -> 116.9 ms.
 template <int N, int R, int G>
 __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const double (&y)[Cell<N, R, G>::RPL],
                                          const double (&src)[Cell<N, R, G>::RPL], double rhohsrc) {
