@@ -293,9 +293,9 @@ __global__ void gelu_bwd_kernel(long rows, int cols, const float* dA, long lda, 
 // db[c] = sum over rows of d[r, c]: four partial sums of the rows r, r + 4, .., each in row order (the
 // first Adam step divides a bias gradient by its own magnitude, so its rounding is part of the
 // result), then (0 + 1) + (2 + 3). 16 columns per block; 512 threads stage 512 rows in LDS, the next
-// tile's loads in flight while one wavefront adds. What bounds it is that wavefront's chain of
-// additions: 4096 rows of 256 columns 240 us with the adding threads reading memory themselves (64
-// columns per block), 16 us now (9 us with a tree over 64 partial sums, whose rounding shifted the
+// tile's loads in flight while one wavefront adds. What bounds it is the latency of those loads on a
+// few CUs (two smaller tiles in flight 18 us): 4096 rows of 256 columns 240 us with the adding threads
+// reading memory themselves (64 columns per block), 16 us now (9 us with a tree over 64 partial sums, whose rounding shifted the
 // first steps of biases with gradients near Adam's epsilon).
 constexpr int kSumCols = 16, kSumRows = 512;
 __global__ void __launch_bounds__(512) col_sum_kernel(long rows, int cols, const float* d, long ld, float* out,
