@@ -292,6 +292,8 @@ const SizeRule kSizeRules[] = {  // per mechanism in ascending order
     {kAnySize, PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 3)},
 };
 
+constexpr int kNumSizeRules = (int)(sizeof(kSizeRules) / sizeof(kSizeRules[0]));
+
 std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
   prk::BlobLayout L = prk::blob_layout(m->nsp, m->nr, m->neff, m->ninc);
   std::vector<unsigned char> b(L.bytes, 0);
@@ -711,6 +713,13 @@ struct Surrogate {
   std::vector<void*> owned;
 };
 
+// Block, LDS bytes and resident blocks of a BDF kernel (cap 0: not asked for yet).
+struct BdfFit {
+  int block = 0;
+  size_t shmem = 0;
+  long cap = 0;
+};
+
 struct pr_handle {
   // Calls on one handle are serialized (its buffers, counters and statistics are shared state);
   // recursive because entry points call each other (pr_advance_chemistry_box -> pr_react_box).
@@ -732,6 +741,7 @@ struct pr_handle {
   double* d_gscr = nullptr;    // per-group global scratch slots
   size_t gscr_bytes = 0;
   bool use_typ = false;
+  BdfFit fits[kNumSizeRules];  // of the mechanism's size rules
   pr_stats last{};
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr, ev3 = nullptr;
   Surrogate* surr = nullptr;
@@ -890,21 +900,53 @@ static int bdf_block(const pr_handle* h, const Variant* v) {
   return 64;
 }
 
+// Launch shape of a BDF variant in this handle: its block and the most blocks that can be resident.
+static int bdf_fit(pr_handle* h, const Variant* v, BdfFit* f) {
+  f->block = bdf_block(h, v);
+  if (f->block > 256 * v->waves)
+    return fail(PR_ERR_KEY, "hipbdf.block " + std::to_string(f->block) + " exceeds " +
+                                std::to_string(256 * v->waves) + " threads for " + std::to_string(v->G) +
+                                " lanes per cell");
+  f->shmem = (size_t)h->blob_bytes + (size_t)(f->block / v->G) * v->scratch;
+  int dev_cus = 0, nb = 0;
+  HIPCHK(hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, h->device));
+  HIPCHK(v->occ(&nb, f->block, f->shmem));
+  if (nb < 1) return fail(PR_ERR_HIP, "kernel does not fit on a CU with this block / LDS size");
+  f->cap = (long)nb * dev_cus;
+  return 0;
+}
+
+// Blocks of a launch of up to work cells, and the bytes of their global slots.
+static long bdf_blocks(const Variant* v, const BdfFit& f, long work) {
+  const long per = f.block / v->G, want = (work + per - 1) / per;
+  return want < 1 ? 1 : (want < f.cap ? want : f.cap);
+}
+static size_t bdf_slots(const Variant* v, const BdfFit& f, long work) {
+  return (size_t)bdf_blocks(v, f, work) * (size_t)(f.block / v->G) * (size_t)v->slot;
+}
+
 // BDF kernel of a launch of up to work cells: the handle's variant when a key chooses one, else by
-// size. slots: bytes of global slots that smaller launches of the handle may need.
-static const Variant* bdf_variant(const pr_handle* h, long work, int* block, size_t* slots) {
+// size. slots: bytes of global slots that smaller launches of the handle may need, no more than can
+// be resident (a slot is 57 KB for 54 components).
+static int bdf_variant(pr_handle* h, long work, const Variant** var, BdfFit* fit, size_t* slots) {
   const Keys& K = h->keys;
-  const Variant* v = h->var;
   *slots = 0;
-  if (!K.lanes_per_cell && !K.waves && !K.block && !K.autotune)
-    for (const SizeRule& r : kSizeRules)
-      if (std::strcmp(r.v.mech, h->mech->name) == 0) {
-        v = &r.v;
-        if (work <= r.max_cells) break;
-        *slots = std::max(*slots, (size_t)(r.max_cells + 256 * r.v.waves / r.v.G) * (size_t)r.v.slot);
-      }
-  *block = bdf_block(h, v);
-  return v;
+  if (K.lanes_per_cell || K.waves || K.block || K.autotune) {
+    *var = h->var;
+    return bdf_fit(h, h->var, fit);
+  }
+  for (int i = 0; i < kNumSizeRules; ++i) {
+    const SizeRule& r = kSizeRules[i];
+    if (std::strcmp(r.v.mech, h->mech->name) != 0) continue;
+    BdfFit& f = h->fits[i];
+    if (f.cap == 0)
+      if (int rc = bdf_fit(h, &r.v, &f)) return rc;
+    *var = &r.v;
+    *fit = f;
+    if (work <= r.max_cells) break;
+    *slots = std::max(*slots, bdf_slots(&r.v, f, r.max_cells));
+  }
+  return 0;
 }
 
 static int ensure_gscr(pr_handle* h, size_t need) {
@@ -937,34 +979,24 @@ static prk::Arr to_arr(const pr_array4* a) {
 // bytes and the grid is capped to the groups it holds; otherwise the handle's slots grow to fit.
 static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t st, double* gscr = nullptr,
                       size_t gscr_cap = 0) {
-  int block = 0;
+  BdfFit fit;
+  const Variant* v = nullptr;
   size_t smaller = 0;
-  const Variant* v = bdf_variant(h, work_max, &block, &smaller);
-  const int G = v->G;
-  if (block > 256 * v->waves)
-    return fail(PR_ERR_KEY, "hipbdf.block " + std::to_string(block) + " exceeds " + std::to_string(256 * v->waves) +
-                                " threads for " + std::to_string(G) + " lanes per cell");
-  const size_t shmem = (size_t)h->blob_bytes + (size_t)(block / G) * v->scratch;
-  int dev_cus = 0, nb = 0;
-  HIPCHK(hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, h->device));
-  HIPCHK(v->occ(&nb, block, shmem));
-  if (nb < 1) return fail(PR_ERR_HIP, "kernel does not fit on a CU with this block / LDS size");
-  long cap = (long)nb * dev_cus;
+  if (int rc = bdf_variant(h, work_max, &v, &fit, &smaller)) return rc;
+  const int G = v->G, block = fit.block;
+  const size_t shmem = fit.shmem;
   if (gscr) {
     const size_t per = (size_t)(block / G) * (size_t)v->slot;  // 0: a variant without global slots
-    const long fit = per ? (long)(gscr_cap / per) : cap;
-    if (fit < 1) return fail(PR_ERR_ARG, "scratch too small for one block of this kernel variant");
-    cap = fit < cap ? fit : cap;
+    const long room = per ? (long)(gscr_cap / per) : fit.cap;
+    if (room < 1) return fail(PR_ERR_ARG, "scratch too small for one block of this kernel variant");
+    fit.cap = room < fit.cap ? room : fit.cap;
   }
-  long want = (work_max + (block / G) - 1) / (block / G);
-  if (want < 1) want = 1;
-  const int blocks = (int)(want < cap ? want : cap);
+  const int blocks = (int)bdf_blocks(v, fit, work_max);
   if (gscr) {
     P.gscr = gscr;
   } else {
     // a smaller launch may take another variant; it finds its slots allocated, as a captured one has to
-    const size_t need = std::max(smaller, (size_t)blocks * (size_t)(block / G) * (size_t)v->slot);
-    int rc = ensure_gscr(h, need);
+    int rc = ensure_gscr(h, std::max(smaller, bdf_slots(v, fit, work_max)));
     if (rc) return rc;
     P.gscr = h->d_gscr;
   }

@@ -118,3 +118,36 @@ def test_jacobians_by_block(gpu, mech, lanes, cells):
     J = r.jac_batch(dev(y), dev(box["rYsrc"]), dev(box["rHsrc"])).cpu().numpy()
     r.close()
     _bits("jac", J, ref)
+
+
+def _free_after(torch, f):
+    """Bytes of device memory that f() takes."""
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    f()
+    torch.cuda.synchronize()
+    return before - torch.cuda.mem_get_info()[0]
+
+
+# doubles of a group's global slot (saved Jacobian, five records per reaction, LU factors above 32
+# components) times the groups that the waves of the rules up to this size can hold
+@pytest.mark.parametrize("mech,cells,slot,groups", [("dodecane_lu", 6145, 2 * 54 * 54 + 5 * 253, 4 * 3),
+                                                    ("LiDryer", 28673, 10 * 10 + 5 * 21, 4 * 4 * 64 // 16)])
+def test_slots_of_what_can_be_resident(gpu, mech, cells, slot, groups):
+    """A launch reserves slots for the groups that can run at once, not for the cells of a smaller rule."""
+    import torch
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    t = box_tensors(BOXES[mech](nx=cells, ny=1, nz=1, dt=1e-9), gpu)
+
+    def react(r):
+        r.react(t["rY"], t["rYsrc"], t["T"], t["rH"], t["rHsrc"], t["FC"], t["mask"], 1e-9, 0.0)
+
+    rs = [Reactor.create("ReactorCvode", mech, KEYS) for _ in range(2)]
+    for r in rs:
+        r.init(2, 1)
+    react(rs[0])  # the kernels' own memory
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    taken = _free_after(torch, lambda: react(rs[1]))
+    for r in rs:
+        r.close()
+    assert taken <= 8 * slot * groups * cus + (8 << 20)  # tables and cost order: a few pages of 2 MiB
