@@ -210,9 +210,13 @@ struct Variant {
 // registers already spill at 2. LiDryer at 16 lanes fits 3 waves without spills (21% faster than
 // 2 on a 32^3 box); at 8 lanes 4 waves spill and are slower. A 54-component state (syn53) keeps
 // its LU factors in its global slot too: 223 VGPRs at 2 waves (no spills), 45 spilled at 3.
+// The first of a mechanism at its default lanes is the one a handle has without keys.
 const Variant kVariants[] = {
     PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 3),
     PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 8, 2),
+    PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 64, 2),
+    PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 32, 3),
+    PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 4),
     PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 32, 4),
     PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 32, 3),
     PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 16, 2),
@@ -222,6 +226,7 @@ const Variant kVariants[] = {
     PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 2),
     PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 3),
 };
+constexpr int kNumVariants = (int)(sizeof(kVariants) / sizeof(kVariants[0]));
 
 // Lanes per cell of the block kernels (block_rates.h): a quad up to 32 components, 8 lanes above.
 constexpr int block_lanes(int n) { return n <= 32 ? 4 : 8; }
@@ -275,24 +280,17 @@ const Variant* find_variant(const char* mech, int G, int W = 0) {
 //   52.5 / 39.0, 8000 66.0 / 44.6 against 62.2 / 38.9, 32768 200 / 175 against 174 / 148. syn53: 4096
 //   29.5 / 20.8 against 28.0 / 21.9, 13824 62.1 / 48.7 against 57.2 / 42.2.
 struct SizeRule {
+  const char* mech;
   long max_cells;
-  Variant v;
+  int G, waves;  // of kVariants
 };
 constexpr long kAnySize = 1L << 62;
 const SizeRule kSizeRules[] = {  // per mechanism in ascending order
-    {2048, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 64, 2)},
-    {7168, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 32, 3)},
-    {28672, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 3)},
-    {kAnySize, PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 4)},
-    {6144, PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 64, 2)},
-    {kAnySize, PR_VARIANT("drm19", PR_DRM19_NSP, PR_DRM19_NR, 32, 4)},
-    {6144, PR_VARIANT("syn53", PR_SYN53_NSP, PR_SYN53_NR, 64, 2)},
-    {kAnySize, PR_VARIANT("syn53", PR_SYN53_NSP, PR_SYN53_NR, 64, 3)},
-    {6144, PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 2)},
-    {kAnySize, PR_VARIANT("dodecane_lu", PR_DODECANE_LU_NSP, PR_DODECANE_LU_NR, 64, 3)},
+    {"LiDryer", 2048, 64, 2},      {"LiDryer", 7168, 32, 3},      {"LiDryer", 28672, 16, 3},
+    {"LiDryer", kAnySize, 16, 4},  {"drm19", 6144, 64, 2},        {"drm19", kAnySize, 32, 4},
+    {"syn53", 6144, 64, 2},        {"syn53", kAnySize, 64, 3},    {"dodecane_lu", 6144, 64, 2},
+    {"dodecane_lu", kAnySize, 64, 3},
 };
-
-constexpr int kNumSizeRules = (int)(sizeof(kSizeRules) / sizeof(kSizeRules[0]));
 
 std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
   prk::BlobLayout L = prk::blob_layout(m->nsp, m->nr, m->neff, m->ninc);
@@ -741,7 +739,8 @@ struct pr_handle {
   double* d_gscr = nullptr;    // per-group global scratch slots
   size_t gscr_bytes = 0;
   bool use_typ = false;
-  BdfFit fits[kNumSizeRules];  // of the mechanism's size rules
+  bool pinned = false;  // a key or the autotuner chose var / block: no rule by size
+  BdfFit fits[kNumVariants];  // of the variants the size rules name
   pr_stats last{};
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr, ev3 = nullptr;
   Surrogate* surr = nullptr;
@@ -802,6 +801,7 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
   h->var = v;
   h->keys = K;
   h->block = K.block;
+  h->pinned = K.lanes_per_cell || K.waves || K.block;
   hipError_t e = hipGetDevice(&h->device);
   if (e != hipSuccess) {
     delete h;
@@ -929,22 +929,21 @@ static size_t bdf_slots(const Variant* v, const BdfFit& f, long work) {
 // size. slots: bytes of global slots that smaller launches of the handle may need, no more than can
 // be resident (a slot is 57 KB for 54 components).
 static int bdf_variant(pr_handle* h, long work, const Variant** var, BdfFit* fit, size_t* slots) {
-  const Keys& K = h->keys;
   *slots = 0;
-  if (K.lanes_per_cell || K.waves || K.block || K.autotune) {
+  if (h->pinned) {
     *var = h->var;
     return bdf_fit(h, h->var, fit);
   }
-  for (int i = 0; i < kNumSizeRules; ++i) {
-    const SizeRule& r = kSizeRules[i];
-    if (std::strcmp(r.v.mech, h->mech->name) != 0) continue;
-    BdfFit& f = h->fits[i];
+  for (const SizeRule& r : kSizeRules) {
+    if (std::strcmp(r.mech, h->mech->name) != 0) continue;
+    const Variant* v = find_variant(r.mech, r.G, r.waves);
+    BdfFit& f = h->fits[v - kVariants];
     if (f.cap == 0)
-      if (int rc = bdf_fit(h, &r.v, &f)) return rc;
-    *var = &r.v;
+      if (int rc = bdf_fit(h, v, &f)) return rc;
+    *var = v;
     *fit = f;
     if (work <= r.max_cells) break;
-    *slots = std::max(*slots, bdf_slots(&r.v, f, r.max_cells));
+    *slots = std::max(*slots, bdf_slots(v, f, r.max_cells));
   }
   return 0;
 }
@@ -1168,7 +1167,8 @@ static int mlp_forward(pr_handle* h, long ncells, hipStream_t st) {
 // hipbdf.autotune: on the first react call, every lanes-per-cell variant of the mechanism, with
 // its own block size and with 128 and 256 threads, integrates the same evenly spaced sample (up to 65536
 // cells) of the box (a copy:
-// the box itself is untouched); the fastest per cell is kept for the handle. All variants give
+// the box itself is untouched); the fastest per cell is kept for the handle, whatever the size of
+// later launches. All variants give
 // identical results, so the choice only affects speed.
 static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc& B, hipStream_t st) {
   if (!h->keys.autotune || h->tuned) return 0;
@@ -1177,7 +1177,7 @@ static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc&
   // the sample must be many times the cells resident on the GPU at once, or the launch tail
   // (not the steady state) decides the ranking
   const long S = B.ncells < 65536 ? B.ncells : 65536;
-  if (S < 4096) return 0;  // too small to tell variants apart
+  if (S < 4096) return 0;  // too small to tell variants apart: the choice stays as without the key
   double* buf = nullptr;
   const size_t per = (size_t)(2 * N + 4);
   HIPCHK(hipMalloc(&buf, sizeof(double) * S * per * 2));
@@ -1213,6 +1213,8 @@ static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc&
   std::vector<long> starts = {0L, S};
   const Variant* v0 = h->var;
   const int b0 = h->block;
+  const bool p0 = h->pinned;
+  h->pinned = true;
   for (const Variant& v : kVariants) {
     if (e != hipSuccess) break;
     if (std::strcmp(v.mech, h->mech->name) != 0) continue;
@@ -1256,6 +1258,7 @@ static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc&
   (void)hipFree(buf);
   h->var = (e == hipSuccess) ? best_v : v0;
   h->block = (e == hipSuccess) ? best_b : b0;
+  h->pinned = e == hipSuccess || p0;
   if (e != hipSuccess) return fail(PR_ERR_HIP, std::string("autotune: ") + hipGetErrorString(e));
   return 0;
 }

@@ -120,6 +120,46 @@ def test_jacobians_by_block(gpu, mech, lanes, cells):
     _bits("jac", J, ref)
 
 
+@pytest.mark.parametrize("lanes,waves", [(64, 2), (32, 3), (16, 4)])
+def test_rule_variants_by_key(gpu, lanes, waves):
+    """What the size rules launch can be chosen by key too, with the same bits."""
+    import torch
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    box = W.h2_air_box(nx=67, ny=1, nz=1)
+    out = []
+    for keys in ({"hipbdf.lanes_per_cell": 8}, {"hipbdf.lanes_per_cell": lanes, "hipbdf.waves_per_simd": waves}):
+        r = Reactor.create("ReactorCvode", "LiDryer", dict(KEYS, **keys))
+        r.init(2, 1)
+        t = box_tensors(box, gpu)
+        r.react(t["rY"], t["rYsrc"], t["T"], t["rH"], t["rHsrc"], t["FC"], t["mask"], box["dt"], 0.0)
+        torch.cuda.synchronize()
+        out.append({k: t[k].cpu().numpy() for k in ("rY", "T", "rH", "FC")})
+        st = r.stats()
+        t = box_tensors(box, gpu)  # the other kernels of the handle take its lanes as well
+        y = torch.cat([t["rY"].reshape(-1, 67), t["T"].reshape(1, 67)]).contiguous()
+        src, rHsrc = t["rYsrc"].reshape(-1, 67).contiguous(), t["rHsrc"].reshape(67)
+        out[-1]["rhs"] = r.rhs_batch(y, src, t["rH"].reshape(67), rHsrc).cpu().numpy()
+        out[-1]["jac"] = r.jac_batch(y, src, rHsrc).cpu().numpy()
+        out[-1]["rates"] = r.reaction_rate_rhoY(t["rY"] * 1e3, t["rH"] * 0.1, t["T"]).cpu().numpy()
+        r.close()
+    assert (st["lanes_per_cell"], st["waves_per_simd"]) == (lanes, waves)
+    for k in out[0]:
+        _bits(k, out[1][k], out[0][k])
+
+
+def test_autotune_leaves_small_boxes_to_the_size_rules(gpu):
+    """A first box too small to tell variants apart chooses none: the launch is the one without the key."""
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    box = W.h2_air_box(nx=100, ny=1, nz=1)
+    r = Reactor.create("ReactorCvode", "LiDryer", dict(KEYS, **{"hipbdf.autotune": 1}))
+    r.init(2, 1)
+    t = box_tensors(box, gpu)
+    r.react(t["rY"], t["rYsrc"], t["T"], t["rH"], t["rHsrc"], t["FC"], t["mask"], box["dt"], 0.0)
+    st = r.stats()
+    r.close()
+    assert (st["lanes_per_cell"], st["waves_per_simd"]) == (64, 2)
+
+
 def _free_after(torch, f):
     """Bytes of device memory that f() takes."""
     torch.cuda.synchronize()
