@@ -926,24 +926,35 @@ static size_t bdf_slots(const Variant* v, const BdfFit& f, long work) {
 }
 
 // BDF kernel of a launch of up to work cells: the handle's variant when a key chooses one, else by
-// size. slots: bytes of global slots that smaller launches of the handle may need, no more than can
-// be resident (a slot is 57 KB for 54 components).
+// size. slots: bytes of global slots that other launches of the handle may need, which a captured
+// one cannot allocate: those of smaller launches and, once a launch has filled the mechanism's
+// default variant, those of every launch. No more than can be resident (a slot is 57 KB for 54
+// components).
 static int bdf_variant(pr_handle* h, long work, const Variant** var, BdfFit* fit, size_t* slots) {
   *slots = 0;
   if (h->pinned) {
     *var = h->var;
     return bdf_fit(h, h->var, fit);
   }
+  auto fit_of = [&](const Variant* v, const BdfFit** f) {
+    BdfFit& k = h->fits[v - kVariants];
+    *f = &k;
+    return k.cap == 0 ? bdf_fit(h, v, &k) : 0;
+  };
+  const BdfFit* f = nullptr;
+  if (int rc = fit_of(h->var, &f)) return rc;
+  const bool full = work >= f->cap * (f->block / h->var->G);
+  *var = nullptr;
   for (const SizeRule& r : kSizeRules) {
     if (std::strcmp(r.mech, h->mech->name) != 0) continue;
     const Variant* v = find_variant(r.mech, r.G, r.waves);
-    BdfFit& f = h->fits[v - kVariants];
-    if (f.cap == 0)
-      if (int rc = bdf_fit(h, v, &f)) return rc;
-    *var = v;
-    *fit = f;
-    if (work <= r.max_cells) break;
-    *slots = std::max(*slots, bdf_slots(v, f, r.max_cells));
+    if (int rc = fit_of(v, &f)) return rc;
+    if (!*var && work <= r.max_cells) {
+      *var = v;
+      *fit = *f;
+    }
+    if (full || !*var) *slots = std::max(*slots, bdf_slots(v, *f, r.max_cells));
+    else break;
   }
   return 0;
 }
@@ -994,7 +1005,6 @@ static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t 
   if (gscr) {
     P.gscr = gscr;
   } else {
-    // a smaller launch may take another variant; it finds its slots allocated, as a captured one has to
     int rc = ensure_gscr(h, std::max(smaller, bdf_slots(v, fit, work_max)));
     if (rc) return rc;
     P.gscr = h->d_gscr;

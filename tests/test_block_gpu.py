@@ -191,3 +191,44 @@ def test_slots_of_what_can_be_resident(gpu, mech, cells, slot, groups):
     for r in rs:
         r.close()
     assert taken <= 8 * slot * groups * cus + (8 << 20)  # tables and cost order: a few pages of 2 MiB
+
+
+# the cells that fill the default variant (groups of its waves on 256 CUs), and one past the last line
+@pytest.mark.parametrize("mech,small,large", [("dodecane_lu", 4 * 2 * 256, 6145),
+                                              ("LiDryer", 4 * 3 * 64 // 16 * 256, 28673)])
+def test_larger_launches_find_their_slots(gpu, mech, small, large):
+    """After a launch that fills the default variant a larger one allocates no slots, so it can be captured."""
+    import torch
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    dt = 1e-9
+    rs = [Reactor.create("ReactorCvode", mech, dict(KEYS, **{"hipbdf.cost_order": 0})) for _ in range(2)]
+    tl, ts = (dict(box_tensors(BOXES[mech](nx=n, ny=1, nz=1, dt=dt), gpu), dt=dt) for n in (large, small))
+    pristine = {k: tl[k].clone() for k in ("rY", "T", "rH", "FC")}
+
+    def restore():
+        for k, v in pristine.items():
+            tl[k].copy_(v)
+
+    for r in rs:
+        r.init(2, 1)
+    for t in (tl, ts):  # the kernels' own memory
+        rs[0].react_batch([t])
+    ref = {k: tl[k].clone() for k in pristine}
+    r = rs[1]
+    r.react_batch([ts])
+    assert _free_after(torch, lambda: r.react_batch([tl])) <= 4 << 20
+    r.close()
+    r = Reactor.create("ReactorCvode", mech, dict(KEYS, **{"hipbdf.cost_order": 0}))
+    r.init(2, 1)
+    r.react_batch([ts])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        r.react_batch([tl], enqueue_only=True)
+    for _ in range(3):
+        restore()
+        g.replay()
+        assert r.collect() == 0
+        for k, v in ref.items():
+            assert torch.equal(tl[k], v), k
+    r.close()
+    rs[0].close()
