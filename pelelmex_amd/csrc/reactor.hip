@@ -1474,7 +1474,10 @@ static int audit_launch(pr_handle* h, const prk::KParams& P, const prk::BoxDesc&
   A.queue = reinterpret_cast<unsigned int*>(base + 128);
   A.nfail = reinterpret_cast<unsigned int*>(base + 132);
   A.stats = reinterpret_cast<unsigned long long*>(base + 192);
+  // pr_stats describes the main launch: the audit's is smaller and may be another variant
+  const pr_stats main_launch = h->last;
   if (int rc = bdf_launch(h, A, acap, st)) return rc;
+  h->last = main_launch;
   hipLaunchKernelGGL(prk::audit_err_kernel, dim3(grid), dim3(128), 0, st, N, &S->cnt[1], acap, adesc.rY.p,
                      adesc.T.p, S->aud_out, S->aud_err);
   HIPCHK(hipGetLastError());

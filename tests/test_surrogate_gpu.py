@@ -243,3 +243,27 @@ def test_batch_with_learned_map_graph_replay(gpu):
             for k in rf:
                 np.testing.assert_array_equal(t[k].cpu().numpy(), rf[k].cpu().numpy(), err_msg=f"replay {rep} {k}")
     r.close()
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_stats_describe_the_main_launch(gpu, batch):
+    """The launch shape in pr_stats is the fallback integration's, not the small audit's after it."""
+    import torch
+    from pelelmex_amd import surrogate as sg
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    model = _model()
+    box = W.ch4_air_flame_box(nx=32, ny=16, nz=16, seed=5, dt=5e-6)  # above the line of the 64-lane variant
+    r = Reactor.create("ReactorCvode", "drm19", _keys(model, **{"surrogate.audit_frac": 0.05}))
+    r.init(2, 1)
+    sg.attach(r, model)
+    t = box_tensors(box, gpu)
+    if batch:
+        r.react_batch([dict(t, dt=box["dt"])])
+    else:
+        r.react(t["rY"], t["rYsrc"], t["T"], t["rH"], t["rHsrc"], t["FC"], t["mask"], box["dt"], 0.0)
+    torch.cuda.synchronize()
+    st = r.stats()
+    r.close()
+    assert 0 < st["sur_audited"] < 6144
+    assert (st["lanes_per_cell"], st["waves_per_simd"], st["block_threads"]) == (32, 4, 1024)
+    assert st["blocks"] == 8192 // 32
