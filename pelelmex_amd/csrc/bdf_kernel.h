@@ -188,9 +188,18 @@ __device__ __forceinline__ ExpK exp_constants() {
               kc(1.0 / 720.0),      kc(1.0 / 120.0),      kc(1.0 / 24.0),      kc(1.0 / 6.0)};
 }
 
+// v to an int, saturated (NaN: 0), as the instruction does it; the language's conversion is undefined
+// where the value does not fit.
+__device__ __forceinline__ int int_sat(double v) {
+  int r;
+  asm("v_cvt_i32_f64 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
 // M exponentials at once, the bits of pr_exp: M independent chains in one basic block (one chain of
 // 20 dependent FP64 operations leaves most issue slots of a wavefront empty). pr_exp's range tests
-// are one comparison per argument and a branch no wavefront takes in practice.
+// are one comparison per argument and a branch that only extreme arguments take: Troe fits with
+// T*** = 1e-30 (LiDryer and dodecane_lu have such) give -T / T*** near -1e33 in every cell.
 template <int M>
 __device__ __forceinline__ void exp_n(const ExpK& K, const double (&x)[M], double (&e)[M]) {
   bool far = false;
@@ -221,7 +230,7 @@ __device__ __forceinline__ void exp_n(const ExpK& K, const double (&x)[M], doubl
   PRK_EXP_STEP(1.0);
 #undef PRK_EXP_STEP
 #pragma unroll
-  for (int m = 0; m < M; ++m) e[m] = ldexp(p[m], (int)k[m]);
+  for (int m = 0; m < M; ++m) e[m] = ldexp(p[m], int_sat(k[m]));
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
 #pragma unroll
     for (int m = 0; m < M; ++m) {
