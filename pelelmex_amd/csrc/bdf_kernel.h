@@ -908,6 +908,7 @@ __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const do
     }
   }
   const double Ctot = gpsum<G, RPL, N>(lane, cc);
+  group_sync();  // the rates read every lane's species (sums through registers order no memory)
   const ExpK K = exp_constants();
 #pragma unroll 1
   for (int m = 0; m < Cell<N, R, G>::RXL; ++m) {
@@ -974,6 +975,7 @@ __device__ __forceinline__ void jac_eval(const Smem<N, R>& S, int lane, const do
   gpsum2<G, RPL, N>(lane, pn, prcp, sn, rcp);
   gpsum2<G, RPL, N>(lane, psd, pcf, sdcp, scf);
   const double fT = (rhohsrc - sn) / rcp;
+  group_sync();  // lane N sums the last column, which the species' lanes wrote
 #pragma unroll
   for (int s = 0; s < RPL; ++s) {
     const int j = lane + G * s;
