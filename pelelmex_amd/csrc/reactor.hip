@@ -107,8 +107,11 @@ hipError_t rates_block_t(const prk::RateParams& P, const prk::BlockTabs& tab, in
   constexpr size_t shmem = rates_block_shmem<N, R, G>();
   static_assert(shmem <= 163840, "LDS of one CU");
   const long rounds = (P.ncells + 63) / 64, cap = (long)cus * (long)(163840 / shmem);
-  hipLaunchKernelGGL((prk::rates_block_kernel<N, R, G>), dim3((unsigned)(rounds < cap ? rounds : cap)), dim3(64 * G),
-                     shmem, st, P, tab);
+  const dim3 grid((unsigned)(rounds < cap ? rounds : cap)), block(64 * G);
+  if (P.has_mask)
+    hipLaunchKernelGGL((prk::rates_block_kernel<N, R, G, true>), grid, block, shmem, st, P, tab);
+  else
+    hipLaunchKernelGGL((prk::rates_block_kernel<N, R, G, false>), grid, block, shmem, st, P, tab);
   return hipGetLastError();
 }
 
@@ -2024,8 +2027,12 @@ int pr_reaction_rate_box(pr_handle* h, const int lo[3], const int hi[3], const p
   // (us per call, groups / blocks): drm19 4096 cells 32 / 51, 13824 51 / 52, 32768 86 / 57, 262144
   // 471 / 222; LiDryer 4096 28 / 31, 13824 34 / 31, 110592 95 / 51; dodecane_lu 1728 44 / 71, 4096
   // 61 / 71, 13824 125 / 73, 110592 747 / 367. The crossing is near 48 cells per CU up to 32
-  // components and 24 above.
-  if (ncells >= (N + 1 <= 32 ? 48L : 24L) * dev_cus) {
+  // components and 24 above. With a mask it depends on what is covered, which the host does not know:
+  // the groups skip covered cells at once, the blocks need 53 (drm19) and 74 us (dodecane_lu) for
+  // however few cells. A slab of 0 / 50 / 90 % covered: drm19 32768 cells groups 82 / 55 / 40, blocks
+  // 59 / 54 / 53, 64000 137 / 83 / 48 and 83 / 59 / 53; dodecane_lu 21952 173 / 111 / 61 and 124 / 76 / 75,
+  // 32768 239 / 152 / 76 and 126 / 76 / 75. The line lies where a box of which a tenth is left is about as fast.
+  if (ncells >= (N + 1 <= 32 ? 48L : 24L) * (P.has_mask ? 5 : 1) * dev_cus) {
     HIPCHK(h->blk->rates(P, h->tabs, dev_cus, st));
   } else {
     const int G = h->var->G;
