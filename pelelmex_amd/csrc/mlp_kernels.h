@@ -53,7 +53,10 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
 //   LD_K     k contiguous, 16-byte aligned rows: one 16-byte load per tile
 //   LD_PAIR  x contiguous, 4-byte aligned, even extent: one 4-byte load per k gives rows 2 r and
 //            2 r + 1, which go to the wave's two tiles (tile i holds rows 2 r + i)
-//   LD_ANY   any strides: one 2-byte load per element
+//   LD_ROW   k contiguous at any alignment: one 16-byte load per tile, or where a row may begin between
+//            4-byte words the words and both ends (load8_odd); the last k of a row that do not fill one
+//            by single elements (nothing past the row is read)
+//   LD_ANY   x contiguous: one 2-byte load per element, neighbouring lanes on neighbouring elements
 // Blocks: KS == 1: 4 waves cover 64 x 64 (2 x 2), each over the whole K. KS > 1: KS waves share one
 // 32 x 32 tile, wave w taking the K steps w, w + KS, ..; their partial tiles are added in wave order
 // through LDS. The split is for products with a long K and a small result (weight gradients: K is
@@ -61,10 +64,33 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
 // of the loads, not the matrix cores. Products of a
 // training step (batch 4096, 4 layers of 256), 14 in all: 2790 us with operands staged element by
 // element through LDS and no split, 188 us now (a weight gradient 530 -> 16, a forward layer 36 ->
-// 16, a data gradient 25 -> 9).
+// 16, a data gradient 25 -> 9). Rows at any alignment by single elements were slower than through LDS
+// on large products, where each 2-byte load of a wavefront touches 16 rows (through LDS / by elements /
+// one unaligned 16-byte load / LD_ROW, us): 262144 x 256 x 23 (the features' layer over a 64^3 box) 162 / 197 /
+// 126 / 137, 4096 x 4095 x 4097 2019 / 2732 / 1862 / 1216 and with B by rows too 1921 / 4474 / 3113 / 1611.
 constexpr int GT_K = 32, G_PITCH = 40;
-enum { LD_K = 0, LD_PAIR = 1, LD_ANY = 2 };
+enum { LD_K = 0, LD_PAIR = 1, LD_ROW = 2, LD_ANY = 3 };
 constexpr int kSplitWaves = 16;
+
+// Eight elements from an address that may be off a 4-byte word by one element, where a 16-byte load is slow
+// (4096^3 by rows: 920 us at even pitches, 3110 at an odd one, 1610 so): the whole words and the
+// elements at both ends.
+__device__ __forceinline__ bf16x8 load8_odd(const __bf16* q) {
+  const bool off = (reinterpret_cast<uintptr_t>(q) & 2) != 0;
+  uint32_t d[3], w[4];
+  uint16_t e0, e6, e7;
+  __builtin_memcpy(d, __builtin_assume_aligned(q + (off ? 1 : 0), 4), 12);
+  __builtin_memcpy(&e0, q, 2);
+  __builtin_memcpy(&e6, q + 6, 2);
+  __builtin_memcpy(&e7, q + 7, 2);
+  w[0] = off ? e0 | d[0] << 16 : d[0];
+  w[1] = off ? d[0] >> 16 | d[1] << 16 : d[1];
+  w[2] = off ? d[1] >> 16 | d[2] << 16 : d[2];
+  w[3] = (off ? d[2] >> 16 : (uint32_t)e6) | (uint32_t)e7 << 16;
+  bf16x8 f;
+  __builtin_memcpy(&f, w, 16);
+  return f;
+}
 
 // Fragments of the wave's two tiles from operand X (element (x, k) at p[x * sx + k * sk]), rows
 // x0 .. x0 + 31, k0 .. k0 + 31. Rows past nx read row nx - 1 (their results are not stored), k past
@@ -94,6 +120,30 @@ __device__ __forceinline__ void load_frags(const __bf16* __restrict__ p, long sx
     for (int j = 0; j < 8; ++j) {
       f[0][j] = k + j < K ? v[j][0] : zero;
       f[1][j] = k + j < K ? v[j][1] : zero;
+    }
+  } else if constexpr (LD == LD_ROW) {
+    const __bf16* q[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = x0 + 16 * i + r;
+      q[i] = p + (long)(x < nx ? x : nx - 1) * sx + k;
+    }
+    if (k + 8 <= K) {
+      if (((sx | (long)(reinterpret_cast<uintptr_t>(p) >> 1)) & 1) == 0) {  // every row 4-byte aligned
+#pragma unroll
+        for (int i = 0; i < 2; ++i) __builtin_memcpy(&f[i], __builtin_assume_aligned(q[i], 4), sizeof(bf16x8));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) f[i] = load8_odd(q[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          f[i][j] = zero;
+          if (k + j < K) f[i][j] = q[i][j];
+        }
     }
   } else {
 #pragma unroll

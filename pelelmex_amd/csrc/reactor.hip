@@ -167,7 +167,7 @@ int gemm_ld(const __bf16* p, long sx, long sk, int nx, int K) {
   const auto at = reinterpret_cast<uintptr_t>(p);
   if (sk == 1 && sx % 8 == 0 && K % 8 == 0 && at % 16 == 0) return prk::LD_K;
   if (sx == 1 && sk % 2 == 0 && nx % 2 == 0 && at % 4 == 0) return prk::LD_PAIR;
-  return prk::LD_ANY;
+  return sk == 1 ? prk::LD_ROW : prk::LD_ANY;
 }
 
 template <int LA, int LB>
@@ -184,6 +184,16 @@ hipError_t gemm_launch_t(const prk::GemmParams& G, hipStream_t st) {
     hipLaunchKernelGGL((prk::gemm_bf16_kernel<LA, LB, 1>), grid, dim3(256), 0, st, G);
   }
   return hipGetLastError();
+}
+
+template <int LA>
+hipError_t gemm_launch_a(const prk::GemmParams& G, int lb, hipStream_t st) {
+  switch (lb) {
+    case prk::LD_K: return gemm_launch_t<LA, prk::LD_K>(G, st);
+    case prk::LD_PAIR: return gemm_launch_t<LA, prk::LD_PAIR>(G, st);
+    case prk::LD_ROW: return gemm_launch_t<LA, prk::LD_ROW>(G, st);
+    default: return gemm_launch_t<LA, prk::LD_ANY>(G, st);
+  }
 }
 
 struct Variant {
@@ -1111,16 +1121,11 @@ static int ensure_surr_buffers(pr_handle* h, long ncells) {
 static hipError_t gemm_launch(const prk::GemmParams& G, hipStream_t st) {
   if (G.M <= 0 || G.N <= 0) return hipSuccess;
   const int la = gemm_ld(G.A, G.sam, G.sak, G.M, G.K), lb = gemm_ld(G.B, G.sbn, G.sbk, G.N, G.K);
-  switch (3 * la + lb) {
-    case 3 * prk::LD_K + prk::LD_K: return gemm_launch_t<prk::LD_K, prk::LD_K>(G, st);
-    case 3 * prk::LD_K + prk::LD_PAIR: return gemm_launch_t<prk::LD_K, prk::LD_PAIR>(G, st);
-    case 3 * prk::LD_K + prk::LD_ANY: return gemm_launch_t<prk::LD_K, prk::LD_ANY>(G, st);
-    case 3 * prk::LD_PAIR + prk::LD_K: return gemm_launch_t<prk::LD_PAIR, prk::LD_K>(G, st);
-    case 3 * prk::LD_PAIR + prk::LD_PAIR: return gemm_launch_t<prk::LD_PAIR, prk::LD_PAIR>(G, st);
-    case 3 * prk::LD_PAIR + prk::LD_ANY: return gemm_launch_t<prk::LD_PAIR, prk::LD_ANY>(G, st);
-    case 3 * prk::LD_ANY + prk::LD_K: return gemm_launch_t<prk::LD_ANY, prk::LD_K>(G, st);
-    case 3 * prk::LD_ANY + prk::LD_PAIR: return gemm_launch_t<prk::LD_ANY, prk::LD_PAIR>(G, st);
-    default: return gemm_launch_t<prk::LD_ANY, prk::LD_ANY>(G, st);
+  switch (la) {
+    case prk::LD_K: return gemm_launch_a<prk::LD_K>(G, lb, st);
+    case prk::LD_PAIR: return gemm_launch_a<prk::LD_PAIR>(G, lb, st);
+    case prk::LD_ROW: return gemm_launch_a<prk::LD_ROW>(G, lb, st);
+    default: return gemm_launch_a<prk::LD_ANY>(G, lb, st);
   }
 }
 

@@ -163,6 +163,62 @@ def test_gemm_long_k(gpu, a_kfast, b_kfast, M, N, K):
         assert np.all(np.abs(C.cpu().numpy() - Ab @ Bb) <= tol)
 
 
+# rows of k at any alignment: every remainder of a 16-byte load, one and several K steps, split and not
+@pytest.mark.parametrize("a_rows,b_rows", [(True, True), (True, False), (False, True)])
+@pytest.mark.parametrize("M,N,K", [(65, 33, k) for k in (1, 7, 8, 9, 15, 23, 25, 33, 63)] + [(64, 66, 259), (33, 1, 1029)])
+def test_gemm_rows_at_any_alignment(gpu, a_rows, b_rows, M, N, K):
+    """The bits of the same product with rows padded by zeros to whole aligned 16 bytes, for rows from
+    an even or odd element at an even or odd pitch; what lies between and behind the rows is NaN."""
+    import torch
+    from pelelmex_amd import surrogate as sg
+    g = torch.Generator().manual_seed(K)
+    bias = torch.randn(N, generator=g).to(gpu)
+    pad = (K + 7) // 8 * 8
+
+    def operand(x, rows, ld, off):  # (tensor, stride of x's rows, stride of k); columns of x: x contiguous
+        if not rows:
+            return x.t().contiguous().to(torch.bfloat16).to(gpu), 1, x.shape[0]
+        buf = torch.full((off + x.shape[0] * ld + 8,), float("nan"), dtype=torch.bfloat16)
+        buf[off:off + x.shape[0] * ld].view(x.shape[0], ld)[:, :x.shape[1]] = x.to(torch.bfloat16)
+        return buf.to(gpu)[off:], ld, 1
+
+    def products(a, b, k, ld, off):
+        (A, sam, sak), (B, sbn, sbk) = operand(a, a_rows, ld, off), operand(b, b_rows, ld, off)
+        out = []
+        for bi in (bias, None):
+            C = torch.full((M, N), float("nan"), dtype=torch.float32, device=gpu)
+            sg.gemm(M, N, k, A, sam, sak, B, sbk, sbn, bias=bi, Cf=C, ldc=N)
+            out.append(C)
+        return out
+
+    a, b = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    zeros = lambda x: torch.cat([x, torch.zeros(x.shape[0], pad - K)], 1)
+    want = products(zeros(a), zeros(b), pad, pad, 0)
+    assert all(torch.isfinite(w).all() for w in want)
+    for off, odd in ((0, 0), (0, 1), (1, 0), (1, 1), (2, 1)):
+        for got, w in zip(products(a, b, K, K + (K + odd) % 2, off), want):
+            assert torch.equal(got, w), (off, odd)
+
+
+def test_gemm_odd_rows_cost_no_multiple(gpu):
+    """A product of odd rows takes about the time of the aligned one (0.9; 2.4 by single elements)."""
+    import time
+    import torch
+    from pelelmex_amd import surrogate as sg
+    took = []
+    for M, N, K in ((2048, 2048, 2048), (2048, 2047, 2049)):
+        A, B = (torch.randn(n * K, device=gpu).to(torch.bfloat16) for n in (M, N))
+        C, bias, ts = torch.empty((M, N), device=gpu), torch.zeros(N, device=gpu), []
+        for _ in range(20):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            sg.gemm(M, N, K, A, K, 1, B, 1, K, bias=bias, Cf=C, ldc=N)
+            torch.cuda.synchronize()
+            ts.append(time.perf_counter() - t0)
+        took.append(float(np.median(ts)))
+    assert took[1] < 1.6 * took[0]
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (511, 15), (512, 16), (513, 17), (4097, 22), (1030, 256)])
 def test_column_sum(gpu, rows, cols):
     """Four partial sums over rows r, r + 4, .. in row order, then (0 + 1) + (2 + 3): bit for bit."""
