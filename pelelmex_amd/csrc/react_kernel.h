@@ -89,6 +89,7 @@ __global__ void __launch_bounds__(256 * W) __attribute__((amdgpu_waves_per_eu(W,
   constexpr int n = N + 1;
   constexpr int RPL = Cell<N, R, G>::RPL;
   constexpr int Q = QMAXC;
+  if (P.ncells_dev && *P.ncells_dev == 0u) return;  // the variant of two that got no cells: the queue stays
   extern __shared__ __align__(16) unsigned char smem[];
   {
     const uint4* srcb = reinterpret_cast<const uint4*>(P.blob);
@@ -1081,6 +1082,30 @@ __global__ void cost_scan_kernel(unsigned int* hist) {
       a += hist[b];
     }
   }
+}
+
+// Whether a launch of n cells goes to the variant that holds `resident` of them at once (pick[0] = n)
+// or to one that holds all and takes `ratio` times as long for a cell (pick[1] = n), from the cost
+// buckets. The first takes about as long as its most expensive cell, the sum of all over its
+// groups, or, as the groups take cells in cost order, j + 1 cells of the cost at rank j resident;
+// the other as long as the most expensive cell. Costs nobody knows yet (FC all zero): the first.
+__global__ void cost_pick_kernel(const unsigned int* hist, const int* list, const unsigned int* nlist, long nmax,
+                                 long resident, double ratio, unsigned int* pick) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  double most = 0.0, sum = 0.0, rounds = 0.0;
+  long seen = 0, j = 1;
+  for (int b = 0; b < COST_BUCKETS; ++b) {
+    if (hist[b] == 0u) continue;
+    const int key = COST_BUCKETS - 1 - b;
+    const double c = ldexp(1.0 + 0.25 * (key & 3), key >> 2);  // FC + 1, rounded down to a bucket
+    if (most == 0.0) most = c;
+    sum += c * hist[b];
+    for (seen += hist[b]; seen > j * resident; ++j) rounds = fmax(rounds, (j + 1) * c);
+  }
+  const unsigned int n = (unsigned int)cost_count(list, nlist, nmax);
+  const bool other = most > 1.0 && fmax(rounds, sum / resident) > ratio * most;
+  pick[0] = other ? 0u : n;
+  pick[1] = other ? n : 0u;
 }
 
 // Each block counts its cells per bucket in LDS, reserves one range per bucket from the global

@@ -292,17 +292,24 @@ const Variant* find_variant(const char* mech, int G, int W = 0) {
 //  dodecane_lu, 2 waves against 3: 512 cells 36.2 / 31.4 against 37.7 / 34.5, 5832 53.8 / 36.5 against
 //   52.5 / 39.0, 8000 66.0 / 44.6 against 62.2 / 38.9, 32768 200 / 175 against 174 / 148. syn53: 4096
 //   29.5 / 20.8 against 28.0 / 21.9, 13824 62.1 / 48.7 against 57.2 / 42.2.
+// Those boxes have a stiff tail. Where all cells cost the same a variant that cannot hold them at once
+// takes whole rounds: 64 lanes against 32 on 4096 / 6144 drm19 cells in the same burnt state 3.75 / 5.59
+// against 3.54 / 3.62 ms, LiDryer 32 lanes against 16 on 7168 2.39 against 2.07. So with the cost order and
+// known costs, a launch past a rule's resident cells takes the next rule's variant where the costs say so
+// (cost_pick_kernel); ratio is the next variant's time for one cell over the rule's (drm19 2.22 against
+// 1.25 ms, 3.44 against 1.91, 1.42 against 0.83), 0 where the next variant never was the faster one.
 struct SizeRule {
   const char* mech;
   long max_cells;
   int G, waves;  // of kVariants
+  double ratio;
 };
 constexpr long kAnySize = 1L << 62;
 const SizeRule kSizeRules[] = {  // per mechanism in ascending order
-    {"LiDryer", 2048, 64, 2},      {"LiDryer", 7168, 32, 3},      {"LiDryer", 28672, 16, 3},
-    {"LiDryer", kAnySize, 16, 4},  {"drm19", 6144, 64, 2},        {"drm19", kAnySize, 32, 4},
-    {"syn53", 6144, 64, 2},        {"syn53", kAnySize, 64, 3},    {"dodecane_lu", 6144, 64, 2},
-    {"dodecane_lu", kAnySize, 64, 3},
+    {"LiDryer", 2048, 64, 2, 0.0},      {"LiDryer", 7168, 32, 3, 1.1},      {"LiDryer", 28672, 16, 3, 0.0},
+    {"LiDryer", kAnySize, 16, 4, 0.0},  {"drm19", 6144, 64, 2, 1.75},       {"drm19", kAnySize, 32, 4, 0.0},
+    {"syn53", 6144, 64, 2, 0.0},        {"syn53", kAnySize, 64, 3, 0.0},    {"dodecane_lu", 6144, 64, 2, 0.0},
+    {"dodecane_lu", kAnySize, 64, 3, 0.0},
 };
 
 std::vector<unsigned char> pack_blob(const pr_mech_t* m) {
@@ -731,6 +738,19 @@ struct BdfFit {
   long cap = 0;
 };
 
+// A BDF launch: its variant, the one that may be taken instead (null: none), and the bytes of global
+// slots that other launches of the handle may need.
+struct BdfPlan {
+  const Variant* v[2] = {nullptr, nullptr};
+  BdfFit fit[2];
+  double ratio = 0.0;
+  size_t slots = 0;
+};
+
+struct LaunchShape {
+  int lanes = 0, blocks = 0, block = 0, waves = 0;
+};
+
 struct pr_handle {
   // Calls on one handle are serialized (its buffers, counters and statistics are shared state);
   // recursive because entry points call each other (pr_advance_chemistry_box -> pr_react_box).
@@ -748,12 +768,14 @@ struct pr_handle {
   prk::BlockTabs tabs{};       // device tables of the block kernels
   prk::JacTabs jtabs{};        // and of the Jacobian
   double* d_atolv = nullptr;
-  void* d_counters = nullptr;  // two regions of 128 B: queue (4 B), nfail (4 B), stats (8 x 8 B at +64)
+  void* d_counters = nullptr;  // two regions of 128 B: queue, nfail, two counts (cost_pick_kernel; 4 B each), stats (8 x 8 B at +64)
   double* d_gscr = nullptr;    // per-group global scratch slots
   size_t gscr_bytes = 0;
   bool use_typ = false;
   bool pinned = false;  // a key or the autotuner chose var / block: no rule by size
   BdfFit fits[kNumVariants];  // of the variants the size rules name
+  LaunchShape shape[2];        // of the last main launch; the second is taken where the costs say so
+  bool picked = false;         // the last main launch had a second one
   pr_stats last{};
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr, ev3 = nullptr;
   Surrogate* surr = nullptr;
@@ -939,15 +961,13 @@ static size_t bdf_slots(const Variant* v, const BdfFit& f, long work) {
 }
 
 // BDF kernel of a launch of up to work cells: the handle's variant when a key chooses one, else by
-// size. slots: bytes of global slots that other launches of the handle may need, which a captured
-// one cannot allocate: those of smaller launches and, once a launch has filled the mechanism's
-// default variant, those of every launch. No more than can be resident (a slot is 57 KB for 54
-// components).
-static int bdf_variant(pr_handle* h, long work, const Variant** var, BdfFit* fit, size_t* slots) {
-  *slots = 0;
+// size. Slots for other launches are reserved because a captured one cannot allocate them: those of
+// smaller launches and, once a launch has filled the mechanism's default variant, those of every
+// launch. No more than can be resident (a slot is 57 KB for 54 components).
+static int bdf_plan(pr_handle* h, long work, BdfPlan* p) {
   if (h->pinned) {
-    *var = h->var;
-    return bdf_fit(h, h->var, fit);
+    p->v[0] = h->var;
+    return bdf_fit(h, h->var, &p->fit[0]);
   }
   auto fit_of = [&](const Variant* v, const BdfFit** f) {
     BdfFit& k = h->fits[v - kVariants];
@@ -957,17 +977,21 @@ static int bdf_variant(pr_handle* h, long work, const Variant** var, BdfFit* fit
   const BdfFit* f = nullptr;
   if (int rc = fit_of(h->var, &f)) return rc;
   const bool full = work >= f->cap * (f->block / h->var->G);
-  *var = nullptr;
   for (const SizeRule& r : kSizeRules) {
     if (std::strcmp(r.mech, h->mech->name) != 0) continue;
     const Variant* v = find_variant(r.mech, r.G, r.waves);
     if (int rc = fit_of(v, &f)) return rc;
-    if (!*var && work <= r.max_cells) {
-      *var = v;
-      *fit = *f;
+    if (p->v[0] && p->ratio > 0.0 && !p->v[1]) {  // the rule after the launch's
+      p->v[1] = v;
+      p->fit[1] = *f;
     }
-    if (full || !*var) *slots = std::max(*slots, bdf_slots(v, *f, r.max_cells));
-    else break;
+    if (!p->v[0] && work <= r.max_cells) {
+      p->v[0] = v;
+      p->fit[0] = *f;
+      if (h->keys.cost_order && work > f->cap * (f->block / v->G)) p->ratio = r.ratio;
+    } else if (full || !p->v[0]) {
+      p->slots = std::max(p->slots, bdf_slots(v, *f, r.max_cells));
+    }
   }
   return 0;
 }
@@ -997,38 +1021,58 @@ static prk::Arr to_arr(const pr_array4* a) {
 }
 
 // Launches the persistent BDF kernel for up to work_max queue entries; zeroes P.queue, P.stats
-// and P.nfail first (all on the stream).
+// and P.nfail first (all on the stream). A plan with a second variant launches both, each for the
+// number of entries cost_pick_kernel left for it in the words after P.nfail (one of them 0).
 // With gscr given (the no-allocation path), the group slots come from that buffer of gscr_cap
 // bytes and the grid is capped to the groups it holds; otherwise the handle's slots grow to fit.
-static int bdf_launch(pr_handle* h, prk::KParams& P, long work_max, hipStream_t st, double* gscr = nullptr,
-                      size_t gscr_cap = 0) {
-  BdfFit fit;
-  const Variant* v = nullptr;
-  size_t smaller = 0;
-  if (int rc = bdf_variant(h, work_max, &v, &fit, &smaller)) return rc;
-  const int G = v->G, block = fit.block;
-  const size_t shmem = fit.shmem;
-  if (gscr) {
-    const size_t per = (size_t)(block / G) * (size_t)v->slot;  // 0: a variant without global slots
-    const long room = per ? (long)(gscr_cap / per) : fit.cap;
-    if (room < 1) return fail(PR_ERR_ARG, "scratch too small for one block of this kernel variant");
-    fit.cap = room < fit.cap ? room : fit.cap;
+static int bdf_launch(pr_handle* h, prk::KParams& P, const BdfPlan& plan, long work_max, hipStream_t st,
+                      LaunchShape* shape, double* gscr = nullptr, size_t gscr_cap = 0) {
+  const int nv = plan.v[1] ? 2 : 1;
+  size_t need = plan.slots;
+  for (int i = 0; i < nv; ++i) {
+    const Variant* v = plan.v[i];
+    BdfFit fit = plan.fit[i];
+    if (gscr) {
+      const size_t per = (size_t)(fit.block / v->G) * (size_t)v->slot;  // 0: a variant without global slots
+      const long room = per ? (long)(gscr_cap / per) : fit.cap;
+      if (room < 1) return fail(PR_ERR_ARG, "scratch too small for one block of this kernel variant");
+      fit.cap = room < fit.cap ? room : fit.cap;
+    }
+    shape[i] = {v->G, (int)bdf_blocks(v, fit, work_max), fit.block, v->waves};
+    need = std::max(need, bdf_slots(v, fit, work_max));
   }
-  const int blocks = (int)bdf_blocks(v, fit, work_max);
   if (gscr) {
     P.gscr = gscr;
   } else {
-    int rc = ensure_gscr(h, std::max(smaller, bdf_slots(v, fit, work_max)));
+    int rc = ensure_gscr(h, need);
     if (rc) return rc;
     P.gscr = h->d_gscr;
   }
   hipLaunchKernelGGL(prk::zero_counters, dim3(1), dim3(64), 0, st, P.queue, P.stats, P.nfail);
   HIPCHK(hipGetLastError());
-  HIPCHK(v->launch(P, blocks, block, shmem, st));
-  h->last.lanes_per_cell = G;
-  h->last.blocks = blocks;
-  h->last.block_threads = block;
-  h->last.waves_per_simd = v->waves;
+  for (int i = 0; i < nv; ++i) {
+    prk::KParams Q = P;
+    if (nv == 2) Q.ncells_dev = P.nfail + 1 + i;
+    HIPCHK(plan.v[i]->launch(Q, shape[i].blocks, shape[i].block, plan.fit[i].shmem, st));
+  }
+  return 0;
+}
+
+static void set_shape(pr_handle* h, const LaunchShape& s) {
+  h->last.lanes_per_cell = s.lanes;
+  h->last.blocks = s.blocks;
+  h->last.block_threads = s.block;
+  h->last.waves_per_simd = s.waves;
+}
+
+// The launch shape in pr_stats: the main launch's, of its second variant where that one had the cells.
+static int report_shape(pr_handle* h, const unsigned int* nfail, hipStream_t st) {
+  unsigned int n[2] = {0u, 0u};
+  if (h->picked) {
+    HIPCHK(hipMemcpyAsync(n, nfail + 1, sizeof(n), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+  }
+  set_shape(h, h->shape[n[1] > 0 ? 1 : 0]);
   return 0;
 }
 
@@ -1257,7 +1301,10 @@ static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc&
       P.cell_list = nullptr;
       P.ncells_dev = nullptr;
       if ((e = hipEventRecord(h->ev2, st)) != hipSuccess) break;
-      rc = bdf_launch(h, P, S, st);
+      BdfPlan plan;
+      LaunchShape shape[2];
+      rc = bdf_plan(h, S, &plan);
+      if (!rc) rc = bdf_launch(h, P, plan, S, st, shape);
       if (rc) {
         e = hipErrorUnknown;
         break;
@@ -1284,8 +1331,8 @@ static int autotune(pr_handle* h, const prk::KParams& Pbase, const prk::BoxDesc&
 // hipbdf.cost_order: the launch's queue entries (all, or the listed ones) handed out by
 // decreasing input FC, the previous advance's cost; P.cell_list becomes the ordered list (the
 // listed count P.ncells_dev is unchanged). No memset and no allocation once sized for ncells.
-static int cost_order_launch(pr_handle* h, prk::KParams& P, long ncells, hipStream_t st, int* order = nullptr,
-                             unsigned int* hist = nullptr) {
+static int cost_order_launch(pr_handle* h, prk::KParams& P, const BdfPlan& plan, long ncells, hipStream_t st,
+                             int* order = nullptr, unsigned int* hist = nullptr) {
   if (order && hist) {  // the no-allocation path: caller-sized buffers
     hipLaunchKernelGGL(prk::zero_u32, dim3(1), dim3(256), 0, st, hist, 2 * prk::COST_BUCKETS);
   } else if (h->order_cap < ncells) {
@@ -1308,6 +1355,9 @@ static int cost_order_launch(pr_handle* h, prk::KParams& P, long ncells, hipStre
   hipLaunchKernelGGL(prk::cost_hist_kernel, dim3(hgrid), dim3(256), 0, st, P.boxes, P.box_start, P.nbox, list, nlist,
                      ncells, hist);
   hipLaunchKernelGGL(prk::cost_scan_kernel, dim3(1), dim3(64), 0, st, hist);
+  if (plan.v[1])
+    hipLaunchKernelGGL(prk::cost_pick_kernel, dim3(1), dim3(64), 0, st, hist, list, nlist, ncells,
+                       plan.fit[0].cap * (plan.fit[0].block / plan.v[0]->G), plan.ratio, P.nfail + 1);
   hipLaunchKernelGGL(prk::cost_scatter_kernel, dim3(sgrid), dim3(256), 0, st, P.boxes, P.box_start, P.nbox, list,
                      nlist, ncells, hist, order);
   HIPCHK(hipGetLastError());
@@ -1482,10 +1532,11 @@ static int audit_launch(pr_handle* h, const prk::KParams& P, const prk::BoxDesc&
   A.queue = reinterpret_cast<unsigned int*>(base + 128);
   A.nfail = reinterpret_cast<unsigned int*>(base + 132);
   A.stats = reinterpret_cast<unsigned long long*>(base + 192);
-  // pr_stats describes the main launch: the audit's is smaller and may be another variant
-  const pr_stats main_launch = h->last;
-  if (int rc = bdf_launch(h, A, acap, st)) return rc;
-  h->last = main_launch;
+  BdfPlan plan;
+  LaunchShape shape[2];  // pr_stats describes the main launch: the audit's may be another variant
+  if (int rc = bdf_plan(h, acap, &plan)) return rc;
+  plan.v[1] = nullptr;  // its cells are not cost-ordered
+  if (int rc = bdf_launch(h, A, plan, acap, st, shape)) return rc;
   hipLaunchKernelGGL(prk::audit_err_kernel, dim3(grid), dim3(128), 0, st, N, &S->cnt[1], acap, adesc.rY.p,
                      adesc.T.p, S->aud_out, S->aud_err);
   HIPCHK(hipGetLastError());
@@ -1674,19 +1725,22 @@ static int react_box_core(pr_handle* h, const int lo[3], const int hi[3], const 
   P.boxes = dboxes;
   P.box_start = dstart;
   P.nbox = 1;
+  BdfPlan plan;
+  if (int rc = bdf_plan(h, ncells, &plan)) return rc;
+  h->picked = plan.v[1] != nullptr;
   if (h->keys.cost_order) {
-    int rc = fx ? cost_order_launch(h, P, ncells, st, reinterpret_cast<int*>(fx + kFxOrder),
+    int rc = fx ? cost_order_launch(h, P, plan, ncells, st, reinterpret_cast<int*>(fx + kFxOrder),
                                     reinterpret_cast<unsigned int*>(fx + kFxHist))
-                : cost_order_launch(h, P, ncells, st);
+                : cost_order_launch(h, P, plan, ncells, st);
     if (rc) return rc;
   }
   {
     int rc;
     if (fx) {
       const size_t g0 = align256(kFxOrder + (h->keys.cost_order ? sizeof(int) * (size_t)ncells : 0));
-      rc = bdf_launch(h, P, ncells, st, reinterpret_cast<double*>(fx + g0), fx_bytes - g0);
+      rc = bdf_launch(h, P, plan, ncells, st, h->shape, reinterpret_cast<double*>(fx + g0), fx_bytes - g0);
     } else {
-      rc = bdf_launch(h, P, ncells, st);
+      rc = bdf_launch(h, P, plan, ncells, st, h->shape);
     }
     if (rc) return rc;
   }
@@ -1707,6 +1761,7 @@ static int react_box_core(pr_handle* h, const int lo[3], const int hi[3], const 
   HIPCHK(hipEventElapsedTime(&ms_all, h->ev0, h->ev3));
   HIPCHK(hipEventElapsedTime(&ms_sur, h->ev0, h->ev1));
   HIPCHK(hipEventElapsedTime(&ms_bdf, h->ev1, h->ev2));
+  if (int rc = report_shape(h, P.nfail, st)) return rc;
   h->last.cells = (int64_t)hs[0];
   h->last.nst = (int64_t)hs[1];
   h->last.nfe = (int64_t)hs[2];
@@ -1881,13 +1936,17 @@ int pr_react_batch_enqueue(pr_handle* h, int nbox, const pr_box* boxes, void* st
     P.box_start = dstart;
     P.nbox = nbox;
   }
+  BdfPlan plan;
+  if (int rc = bdf_plan(h, total, &plan)) return rc;
+  h->picked = plan.v[1] != nullptr;
   if (h->keys.cost_order) {  // cells of every box by decreasing input FC
-    int rc = cost_order_launch(h, P, total, st);
+    int rc = cost_order_launch(h, P, plan, total, st);
     if (rc) return rc;
   }
   {
-    int rc = bdf_launch(h, P, total, st);
+    int rc = bdf_launch(h, P, plan, total, st, h->shape);
     if (rc) return rc;
+    set_shape(h, h->shape[0]);
   }
   if (audit) {
     int rc = audit_launch(h, P, adesc, dboxes + nbox, dstart + nbox + 1, st);
@@ -1909,13 +1968,8 @@ int pr_collect(pr_handle* h, void* stream) {
   HIPCHK(hipMemcpyAsync(hs, base + 64, sizeof(hs), hipMemcpyDeviceToHost, st));
   HIPCHK(hipMemcpyAsync(&nfail, base + 4, sizeof(nfail), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  const int G = h->last.lanes_per_cell, blocks = h->last.blocks;
-  const int bt = h->last.block_threads, wv = h->last.waves_per_simd;
   h->last = pr_stats{};
-  h->last.lanes_per_cell = G;
-  h->last.blocks = blocks;
-  h->last.block_threads = bt;
-  h->last.waves_per_simd = wv;
+  if (int rc = report_shape(h, reinterpret_cast<unsigned int*>(base + 4), st)) return rc;
   h->last.cells = (int64_t)hs[0];
   h->last.nst = (int64_t)hs[1];
   h->last.nfe = (int64_t)hs[2];

@@ -234,6 +234,65 @@ def test_autotune_leaves_small_boxes_to_the_size_rules(gpu):
     assert (st["lanes_per_cell"], st["waves_per_simd"]) == (64, 2)
 
 
+def _alike(mech, cells, at):
+    """A box of one cell's state, the one at this place in the order of temperatures."""
+    full = BOXES[mech](nx=16, ny=16, nz=16)
+    box = W.subsample(full, np.full(cells, np.argsort(full["T"])[int(at * (full["T"].size - 1))]))
+    if box.get("mask") is not None:
+        box["mask"] = np.ones_like(box["mask"])
+    return box
+
+
+# both sides of what the rule's variant holds at once; cells alike, and a flame whose costs spread widely
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("mech,cells,alike,want", [
+    ("drm19", 2048, True, (64, 2)), ("drm19", 2049, True, (32, 4)), ("drm19", 6144, True, (32, 4)),
+    ("drm19", 4096, False, (64, 2)), ("drm19", 6145, True, (32, 4)), ("LiDryer", 6144, True, (32, 3)),
+    ("LiDryer", 6145, True, (16, 3)), ("LiDryer", 7168, False, (32, 3))])
+def test_variant_by_costs(gpu, mech, cells, alike, want, noalloc):
+    """Where every cell costs the same a launch takes the variant that holds them all at once, from the
+    second call on (the first knows no costs); the bits do not depend on it."""
+    import torch
+    from pelelmex_amd.reactor import Reactor, box_tensors
+    box = _alike(mech, cells, 0.05) if alike else BOXES[mech](nx=cells, ny=1, nz=1)
+    t = box_tensors(box, gpu)
+    old = {k: t[k].clone() for k in ("rY", "T", "rH", "FC")}
+    out = []
+    r = Reactor.create("ReactorCvode", mech, dict(KEYS, **{"cvode.max_order": 4}))
+    r.init(2, 1)
+    for call in range(3):
+        for k in ("rY", "T", "rH"):
+            t[k].copy_(old[k])
+        status = torch.full((cells,), 7, dtype=torch.int32, device=gpu)
+        assert r.react(t["rY"], t["rYsrc"], t["T"], t["rH"], t["rHsrc"], t["FC"], t["mask"], box["dt"], 0.0,
+                       status=status, noalloc=noalloc)[0] == 0
+        torch.cuda.synchronize()
+        assert int(status.abs().sum()) == 0
+        out.append(([t[k].clone() for k in old], r.stats()))
+    shape = lambda st: (st["lanes_per_cell"], st["waves_per_simd"])
+    rule = {"drm19": (64, 2) if cells <= 6144 else (32, 4), "LiDryer": (32, 3)}[mech]
+    assert [shape(st) for _, st in out] == [rule, want, want]
+    assert all(st["cells"] == cells and st["nfe"] == out[0][1]["nfe"] for _, st in out)
+    for got, _ in out[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got, out[0][0]))
+    # and as a batch, captured: the costs of each replay decide
+    if not noalloc:
+        for k in old:
+            t[k].copy_(old[k])
+        r.react_batch([dict(t, dt=box["dt"])])
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            r.react_batch([dict(t, dt=box["dt"])], enqueue_only=True)
+        for first in (True, False, False):
+            for k in old:
+                if k != "FC" or first:
+                    t[k].copy_(old[k])
+            g.replay()
+            assert r.collect() == 0 and shape(r.stats()) == (rule if first else want)
+            assert all(torch.equal(t[k], v) for k, v in zip(old, out[0][0]))
+    r.close()
+
+
 def _free_after(torch, f):
     """Bytes of device memory that f() takes."""
     torch.cuda.synchronize()
