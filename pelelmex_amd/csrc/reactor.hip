@@ -187,9 +187,8 @@ hipError_t gemm_launch_t(const prk::GemmParams& G, hipStream_t st) {
 }
 
 template <int LA>
-hipError_t gemm_launch_a(const prk::GemmParams& G, int lb, hipStream_t st) {
+hipError_t gemm_launch_b(const prk::GemmParams& G, int lb, hipStream_t st) {
   switch (lb) {
-    case prk::LD_K: return gemm_launch_t<LA, prk::LD_K>(G, st);
     case prk::LD_PAIR: return gemm_launch_t<LA, prk::LD_PAIR>(G, st);
     case prk::LD_ROW: return gemm_launch_t<LA, prk::LD_ROW>(G, st);
     default: return gemm_launch_t<LA, prk::LD_ANY>(G, st);
@@ -1164,12 +1163,17 @@ static int ensure_surr_buffers(pr_handle* h, long ncells) {
 
 static hipError_t gemm_launch(const prk::GemmParams& G, hipStream_t st) {
   if (G.M <= 0 || G.N <= 0) return hipSuccess;
-  const int la = gemm_ld(G.A, G.sam, G.sak, G.M, G.K), lb = gemm_ld(G.B, G.sbn, G.sbk, G.N, G.K);
+  int la = gemm_ld(G.A, G.sam, G.sak, G.M, G.K), lb = gemm_ld(G.B, G.sbn, G.sbk, G.N, G.K);
+  // aligned rows beside an operand that is not read in wide loads: the same loads by LD_ROW, four kernels less
+  if (la == prk::LD_K && lb >= prk::LD_ROW) la = prk::LD_ROW;
+  if (lb == prk::LD_K && la >= prk::LD_ROW) lb = prk::LD_ROW;
   switch (la) {
-    case prk::LD_K: return gemm_launch_a<prk::LD_K>(G, lb, st);
-    case prk::LD_PAIR: return gemm_launch_a<prk::LD_PAIR>(G, lb, st);
-    case prk::LD_ROW: return gemm_launch_a<prk::LD_ROW>(G, lb, st);
-    default: return gemm_launch_a<prk::LD_ANY>(G, lb, st);
+    case prk::LD_K: return lb == prk::LD_K ? gemm_launch_t<prk::LD_K, prk::LD_K>(G, st)
+                                           : gemm_launch_t<prk::LD_K, prk::LD_PAIR>(G, st);
+    case prk::LD_PAIR: return lb == prk::LD_K ? gemm_launch_t<prk::LD_PAIR, prk::LD_K>(G, st)
+                                              : gemm_launch_b<prk::LD_PAIR>(G, lb, st);
+    case prk::LD_ROW: return gemm_launch_b<prk::LD_ROW>(G, lb, st);
+    default: return gemm_launch_b<prk::LD_ANY>(G, lb, st);
   }
 }
 
