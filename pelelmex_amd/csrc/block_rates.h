@@ -1,4 +1,5 @@
-// Right-hand sides and rates of 64 cells per block, with the mechanism walked by whole wavefronts.
+// Reaction rates of 64 cells per block, with the mechanism walked by whole wavefronts (and the row sums
+// that setTemperature uses too).
 //
 // A block of 64 G threads (G wavefronts) owns 64 cells and sees them in two layouts:
 //  * rows: a cell belongs to G neighbouring lanes of one wavefront (64 / G cells per wavefront),
@@ -48,7 +49,6 @@ struct BlockTabs {
   const int32_t* rx_range;  // [nchunk * waves + 1] first record of each (chunk, wavefront)
   const GatherPiece* piece;
   const int32_t* piece_range;  // [nchunk * N + 1] first piece of each (chunk, species)
-  int nchunk;
 };
 
 // Sizes of the two layouts for a mechanism.
@@ -101,35 +101,6 @@ __device__ __forceinline__ double rsum(int lane, const double (&a)[BlockCell<N, 
   return t[0];
 }
 
-// Maximum over the group of one value per lane (never NaN).
-template <int G>
-__device__ __forceinline__ double rmax(double v) {
-  v = max_nn(v, dpp_d<0xB1>(v));
-  v = max_nn(v, dpp_d<0x4E>(v));
-  if (G == 8) v = max_nn(v, dpp_d<0x141>(v));
-  return v;
-}
-
-// Value of lane J of the group, J a compile-time constant: quad_perm [J, J, J, J] for quads; for 8
-// lanes the crossbar's swizzle (lane & 0x18) | J.
-template <int G, int J>
-__device__ __forceinline__ double lane_bcast(double v) {
-  if constexpr (G == 4) {
-    return dpp_d<J * 0x55>(v);
-  } else {
-    const int lo = __builtin_amdgcn_ds_swizzle(__double2loint(v), 0x18 | (J << 5));
-    const int hi = __builtin_amdgcn_ds_swizzle(__double2hiint(v), 0x18 | (J << 5));
-    return __hiloint2double(hi, lo);
-  }
-}
-
-// Component K of a vector in the rows layout, to every lane of the group.
-template <int N, int R, int G, int K>
-__device__ __forceinline__ double row_bcast(const double (&a)[BlockCell<N, R, G>::RPL]) {
-  using C = BlockCell<N, R, G>;
-  return lane_bcast<G, (K % C::B) / 2>(a[2 * (K / C::B) + (K & 1)]);
-}
-
 // LDS of the rates: concentrations and g / RT as [species][64 cells] (the gathered production
 // rates later take the concentrations' place), one chunk of rates as [reaction][64], and per-cell
 // T, ln T, 1 / T, ln(R T / P_atm), sum C.
@@ -174,28 +145,21 @@ __device__ __forceinline__ double rows_hy2t(const SpRec* sp, int lane, const dou
   return T;
 }
 
-// The first half of net_rates in the rows layout: everything the cells layout reads goes to LDS
-// (cell: the cell's column), h_k and cp_k stay with their rows.
+// The first half of net_rates in the rows layout: what the cells layout reads goes to LDS (cell: the
+// cell's column).
 template <int N, int R, int G>
 __device__ __forceinline__ void rows_thermo(const RateLds<N, R, G>& L, int lane, int cell, double T,
-                                            const double (&cc)[BlockCell<N, R, G>::RPL],
-                                            double (&hk)[BlockCell<N, R, G>::RPL],
-                                            double (&cpk)[BlockCell<N, R, G>::RPL]) {
+                                            const double (&cc)[BlockCell<N, R, G>::RPL]) {
   using C = BlockCell<N, R, G>;
   const double lnT = pr_log(T), invT = 1.0 / T, lnRTP = pr_log((PR_RU * T) / PR_PATM);
 #pragma unroll
   for (int s = 0; s < C::RPL; ++s) {
     const int i = C::row(lane, s);
-    hk[s] = 0.0;
-    cpk[s] = 0.0;
     if (i < N) {
       double cpR, hRT, gRT, dcp;
       nasa_full(L.sp[i], T, invT, lnT, cpR, hRT, gRT, dcp);
-      const double RW = L.sp[i].RW;
       L.cg[i * C::CELLS + cell] = cc[s];
       L.cg[(N + i) * C::CELLS + cell] = gRT;
-      hk[s] = (hRT * RW) * T;
-      cpk[s] = cpR * RW;
     }
   }
   const double Ctot = rsum<N, R, G, N>(lane, cc);
@@ -485,7 +449,7 @@ __global__ void __launch_bounds__(64 * G) rates_block_kernel(RateParams P, Block
     const int k = P.lo2 + (int)(u / ((unsigned)P.nx * (unsigned)P.ny));
     if (active) {
       const long offY = aoff(P.rY, i, j, k);
-      double ry[C::RPL], Y[C::RPL], cc[C::RPL], hk[C::RPL], cpk[C::RPL];
+      double ry[C::RPL], Y[C::RPL], cc[C::RPL];
 #pragma unroll
       for (int s = 0; s < C::RPL; ++s) {
         const int ii = C::row(lane, s);
@@ -503,7 +467,7 @@ __global__ void __launch_bounds__(64 * G) rates_block_kernel(RateParams P, Block
         const int ii = C::row(lane, s);
         cc[s] = ii < N ? (rho_cgs * Y[s]) * L.sp[ii].invW : 0.0;
       }
-      rows_thermo<N, R, G>(L, lane, cell, T, cc, hk, cpk);
+      rows_thermo<N, R, G>(L, lane, cell, T, cc);
     }
     cells_rates<N, R, G>(L, tab, reinterpret_cast<const int*>(P.blob + BL.off_effsp),
                          reinterpret_cast<const double*>(P.blob + BL.off_effval));

@@ -878,7 +878,6 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
   h->tabs.rx_range = reinterpret_cast<const int32_t*>(h->d_blob + im.tabs[1]);
   h->tabs.piece = reinterpret_cast<const prk::GatherPiece*>(h->d_blob + im.tabs[2]);
   h->tabs.piece_range = reinterpret_cast<const int32_t*>(h->d_blob + im.tabs[3]);
-  h->tabs.nchunk = h->blk->nchunk;
   h->jtabs.term = reinterpret_cast<const prk::JacTerm*>(h->d_blob + im.jtabs[0]);
   h->jtabs.entry = reinterpret_cast<const prk::JacEntry*>(h->d_blob + im.jtabs[1]);
   h->jtabs.slice = reinterpret_cast<const int32_t*>(h->d_blob + im.jtabs[2]);
