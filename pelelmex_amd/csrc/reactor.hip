@@ -846,6 +846,10 @@ int pr_create(const char* integrator, const char* mechanism, int reactor_type, i
     return rc;
   }
   h->blk = find_block_ops(m->name);
+  if (!h->blk) {
+    delete h;
+    return fail(PR_ERR_UNSUPPORTED, std::string("no block kernels (PR_BLOCK_OPS) for mechanism ") + m->name);
+  }
   const MechImage& im = mech_image(m, h->blk);
   h->blob_bytes = im.blob_bytes;
   {
@@ -990,6 +994,10 @@ static int bdf_plan(pr_handle* h, long work, BdfPlan* p) {
     } else if (full || !p->v[0]) {
       p->slots = std::max(p->slots, bdf_slots(v, *f, r.max_cells));
     }
+  }
+  if (!p->v[0]) {  // a mechanism without rules
+    p->v[0] = h->var;
+    p->fit[0] = h->fits[h->var - kVariants];
   }
   return 0;
 }
