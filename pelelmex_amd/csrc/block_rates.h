@@ -11,7 +11,9 @@
 //    through scalar loads, its kind and stoichiometry are scalar branches (no lane of a falloff
 //    or third-body reaction waits for another kind), every lane does useful work, and the
 //    concentrations are read at one stride (conflict-free) from LDS.
-// What bounds it is FP64 VALU issue (two exponentials per reaction). Measured on reactionRateRhoY
+// What bounds it is the latency of each reaction's chain at the three wavefronts per SIMD that 53 KB of LDS
+// per block leave (drm19, 138 VGPRs; one block per CU at 53 species): on 64^3 drm19 cells the SIMDs issue
+// VALU instructions in 52 % of the cycles, 55 % of them FP64 arithmetic. Measured on reactionRateRhoY
 // (rates_block_kernel) against the group kernel's reaction-per-lane form (a record read per lane
 // from LDS, drm19's 84 reactions in three passes of 32 lanes with mixed kinds): 64^3 drm19 cells 471
 // -> 222 us per call, 22533 dodecane_lu cells 186 -> 126 us, the same bits.

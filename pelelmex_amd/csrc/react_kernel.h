@@ -860,7 +860,7 @@ constexpr int eval_jac_doubles() {
 // (MODE 1) for a batch of states stored component-major (y[i * ncells + c]). Up to 32 components a
 // block's Jacobians are assembled in LDS and written out together, an entry of its neighbouring
 // cells at a time: through the global slot every group wrote 8 bytes to each of (N + 1)^2 lines.
-// 8192 drm19 right-hand sides and Jacobians 142 -> 127 us.
+// 8192 drm19 right-hand sides and Jacobians 142 -> 123 us.
 template <int N, int R, int G, int MODE>
 __global__ void __launch_bounds__(BLOCK) eval_kernel(const unsigned char* blob, int blob_bytes, int neff, int ninc,
                                                      long ncells, const double* y, const double* rYsrc,

@@ -219,9 +219,11 @@ struct Variant {
 // instead of 6 KB), which lets 4 waves per SIMD be resident: 32 cells in a 1024-thread block, 44
 // VGPRs spilled, 7 % faster than 3 waves with the factors in LDS (the integrator is latency
 // bound). At 64 lanes the group's LDS does not fit 3 waves; at 16 lanes 4 cells share a wave and
-// registers already spill at 2. LiDryer at 16 lanes fits 3 waves without spills (21% faster than
-// 2 on a 32^3 box); at 8 lanes 4 waves spill and are slower. A 54-component state (syn53) keeps
-// its LU factors in its global slot too: 223 VGPRs at 2 waves (no spills), 45 spilled at 3.
+// 7 registers spill already at 2. LiDryer at 16 lanes: 13 VGPRs spilled at 3 waves (21 % faster than
+// 2 on a 32^3 box), 67 at 4 (the faster one on large boxes all the same, see the size rules); at 32
+// lanes 10 at 3 waves, at 64 none at 2; at 8 lanes 4 waves spill and are slower than 2. A 54-component
+// state keeps its LU factors in its global slot too: no VGPR spilled at 2 waves (208 in use for syn53,
+// 223 for dodecane_lu), 24 and 46 at 3.
 // The first of a mechanism at its default lanes is the one a handle has without keys.
 const Variant kVariants[] = {
     PR_VARIANT("LiDryer", PR_LIDRYER_NSP, PR_LIDRYER_NR, 16, 3),
@@ -2116,7 +2118,8 @@ int pr_reaction_rate_box(pr_handle* h, const int lo[3], const int hi[3], const p
   return 0;
 }
 
-// Launches one of the EOS box kernels (one thread per cell, grid-stride) and synchronizes.
+// Launches one of the EOS box kernels (one thread per cell, setTemperature a quad or eight lanes per cell;
+// grid-stride) and synchronizes.
 static int eos_launch(pr_handle* h, int mode, const int lo[3], const int hi[3], prk::EosParams& P, void* stream) {
   std::lock_guard<std::recursive_mutex> lock(h->mu);
   const long nx = (long)hi[0] - lo[0] + 1, ny = (long)hi[1] - lo[1] + 1, nz = (long)hi[2] - lo[2] + 1;
